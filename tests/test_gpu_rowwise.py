@@ -203,3 +203,36 @@ def test_op_matches_sdpa_like_the_reference(gpu: torch.device) -> None:
     rel = ((out.float() - ref).abs().mean() / ref.abs().mean()).item()
     print(f"scaled-mm mean rel vs SDPA {rel:.4f}", flush=True)
     assert rel < 0.30
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("cols", [8, 504, 520, 2048, 3600, 4096, 4104, 8200, 16384, 16392, 386])
+def test_softmax_rowwise_quantize_widths(gpu: torch.device, cols: int, causal: bool) -> None:
+    """Both softmax kernels around the widths their dispatch divides at: rows
+    in one wave's registers (to 4096 scores), in four waves' (to 16384), longer
+    or not whole 8-score vectors (the three-pass kernel); masked-out, NaN and
+    infinite scores among them.  Same bounds as above: a sum in another order
+    moves a P value by at most one bf16 step, its code by one e4m3 step."""
+    g = torch.Generator().manual_seed(cols + causal)
+    sq = 7
+    raw = (torch.randn(2, sq, cols, generator=g) * 6).to(torch.bfloat16)
+    raw[0, 1] = raw[0, 1, 0]                     # equal scores
+    raw[0, 2, : cols // 2] = float("-inf")       # a half-masked row
+    raw[0, 3, 0] = float("nan")
+    raw[0, 4, 0] = float("inf")                  # inf - inf: a NaN row
+    raw[1, 5] = 1e-30
+    raw[1, 6, cols - 1] = 3e4                    # every other exponential is 0
+    dq, codes = ops.softmax_rowwise_quantize(raw.to(gpu), 0.125, causal)
+    p = rowwise.softmax_probs(raw, 0.125, causal)
+    ref_codes, ref_dq = rowwise.rowwise_quantize(p)
+    d, r = dq.cpu().numpy(), ref_dq.numpy()
+    nan = np.isnan(r)
+    assert np.array_equal(np.isnan(d), nan) and nan[0, 3] and nan[0, 4]
+    assert np.all(np.abs(d - r)[~nan] <= r[~nan] * 2.0 ** -7)
+    gc = codes.view(torch.uint8).cpu().numpy().astype(np.int32)
+    rc = ref_codes.numpy().astype(np.int32)
+    assert ((gc[nan] & 0x7F) == 0x7F).all()
+    assert np.all(np.abs(gc - rc)[~nan] <= 1)
+    # long rows hold few distinct tiny codes near rounding boundaries: the
+    # share of flips stays that of P values at a boundary, as above
+    assert (gc == rc)[~nan].mean() > 0.999
