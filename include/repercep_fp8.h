@@ -448,6 +448,13 @@ int rp_fp8_linear_balanced(const uint8_t* a8, const uint8_t* b8, int b_layout, c
                            const float* b_scale_dev, void* workspace, size_t workspace_bytes,
                            void* stream);
 
+/* Workspace with which rp_fp8_linear_balanced runs a product its own way:
+ * RP_GEMM_BALANCED_WORKSPACE_BYTES, plus the fp32 partial sums of products
+ * whose few rows leave most CUs idle and whose K is therefore split (summed
+ * in a fixed order; with a smaller workspace such a product runs unsplit,
+ * and the two results differ by the order of their fp32 sums). */
+size_t rp_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
 /* rp_fp8_gemm with row-wise scales, batched: for each batch z < `batch`,
  *   C_z (M, N) = bf16( fp32(fp32(A8_z . B8_z) * row_scale_z[m]) * col_scale_z[n] )
  * with A8_z = a8 + z*bsa, B8_z = b8 + z*bsb (bytes), C_z = c + z*bsc,

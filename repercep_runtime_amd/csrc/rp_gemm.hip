@@ -28,6 +28,8 @@
 // Both remap workgroups so that those resident on one XCD cover a compact
 // patch of C and share operand rows in that XCD's L2.
 
+#include <math.h>
+
 #include <type_traits>
 
 #include "rp_common.h"
@@ -61,6 +63,10 @@ struct GemmArgs {
   // counter, zeroed before the launch; null: every tile in place
   unsigned* item_counter;
   int pool_r;
+  // split-K launches of gemm_mid_kernel: fp32 partial sums, part_slices K
+  // slices of 128 per part, (M, N) per part
+  float* part;
+  int part_slices;
 };
 
 // The batch a workgroup works on: offsets every operand pointer (one batch
@@ -812,6 +818,113 @@ int launch_gemm256(GemmArgs g, int64_t batch, hipStream_t st) {
   return RP_OK;
 }
 
+#include "rp_gemm_mid.h"
+
+// Which kernel and tile a product runs on, and over how many K parts.
+struct GemmPlan {
+  int bm = 256;          // 256: gemm256_kernel; 128 or 64: gemm_mid_kernel<bm>
+  int parts = 1;         // K parts (split K)
+  int part_slices = 0;   // 128-byte K slices per part
+};
+
+// The plan of a product that both kernels can run (whole = K % 64 == 0; only
+// the medium tiles take another K), from estimated times in us:
+// * 256 x 256 tiles run in rounds of one per CU: 1.45 per K slice and round
+//   and 4 for a tile's fill and stores (measured 60 for 40 slices);
+// * 128 x 128 tiles: 0.465 per slice and tile of each CU's share, the share
+//   taken as half a tile more than the mean (they run two to a CU), at least
+//   1.25 tiles' time (one alone does not fill the CU);
+// * 64 x 128 tiles 0.32, and better than 128 x 128 only where every tile has
+//   a CU to itself (256 x 5120 x 5120: 21.6 against 22.9 us; 512 rows, 320
+//   tiles: 25.1 against 23.2);
+// * a wave of few tiles waits for its loads, at least 0.45 per slice;
+// * K parts write and read fp32 sums (about 3.5 TB/s) and take another
+//   launch, ~5.5.
+// The constants are fits to a sweep over M 16 .. 16384 of seven projection
+// shapes (a few of its rows stand in rp_gemm_mid.h); where the two kernels'
+// estimates cross they lie within ~4% of each other.
+// A row-scaled (batched) product is never split; nor one whose caller brings
+// no workspace (may_split).
+inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool whole,
+                          bool may_split) {
+  constexpr double kCu = 256.0;
+  const double ns = (double)((K + kG2K - 1) / kG2K);
+  auto tiles = [&](int bm, int bn) {
+    return (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn) * (double)batch;
+  };
+  GemmPlan best;
+  double cost = whole ? ceil(tiles(256, 256) / kCu) * (1.45 * ns + 4.0) : 1e30;
+  for (int bm = 128; bm >= 64; bm -= 64) {
+    const double t = tiles(bm, kGmBN);
+    if (bm == 64 && t > kCu) break;
+    const double c = bm == 128 ? 0.465 : 0.32;
+    for (int parts = 1; parts <= 8; ++parts) {
+      const int per = (int)((ns + parts - 1) / parts);
+      if (parts > 1 && (!may_split || t * parts > 2 * kCu || per < 4 || (per * (parts - 1) >= ns)))
+        break;
+      const double share = fmax(t * parts / kCu, 0.75) + 0.5;
+      double e = per * fmax(c * share, 0.45) + 0.6 * share;
+      if (parts > 1) e += 5.5 + (double)parts * (double)M * (double)N * 8.0 / 3.5e6;
+      if (e < cost) {
+        cost = e;
+        best.bm = bm;
+        best.parts = parts;
+        best.part_slices = per;
+      }
+    }
+  }
+  return best;
+}
+
+// Workspace of rp_fp8_linear_balanced: its item counter, then the K parts.
+inline size_t gemm_workspace_bytes(int64_t M, int64_t N, const GemmPlan& p) {
+  return RP_GEMM_BALANCED_WORKSPACE_BYTES +
+         (p.parts > 1 ? (size_t)p.parts * (size_t)M * (size_t)N * sizeof(float) : 0);
+}
+
+template <int BM, bool KN, int EPI>
+int launch_mid(GemmArgs g, int64_t batch, int parts, hipStream_t st) {
+  g.tiles_m = (int)((g.M + BM - 1) / BM);
+  g.tiles_n = (int)((g.N + kGmBN - 1) / kGmBN);
+  const int64_t nwork = (int64_t)g.tiles_m * g.tiles_n;
+  if (nwork > 0x3fffffff) {
+    rp_set_error("gemm: grid too large");
+    return RP_ERR_UNSUPPORTED;
+  }
+  hipLaunchKernelGGL((gemm_mid_kernel<BM, KN, EPI>),
+                     dim3((unsigned)nwork, (unsigned)batch, (unsigned)parts), dim3(kG2Threads), 0,
+                     st, g);
+  if constexpr (EPI == kEpiPart) {
+    const int64_t threads = g.M * (g.N / 4);
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                       st, g, parts);
+  }
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    rp_set_error("gemm: launch failed: %s", hipGetErrorString(e));
+    return RP_ERR_LAUNCH;
+  }
+  return RP_OK;
+}
+
+template <int BM, bool KN>
+int launch_mid_epi(const GemmArgs& g, int64_t batch, int parts, hipStream_t st) {
+  if (g.row_scale) return launch_mid<BM, KN, kEpiRows>(g, batch, 1, st);
+  if (parts > 1) return launch_mid<BM, KN, kEpiPart>(g, 1, parts, st);
+  if (g.bias) return launch_mid<BM, KN, kEpiBias>(g, 1, 1, st);
+  return launch_mid<BM, KN, kEpiPlain>(g, 1, 1, st);
+}
+
+int launch_gemm_mid(GemmArgs g, int64_t batch, const GemmPlan& p, hipStream_t st) {
+  g.item_counter = nullptr;
+  g.part_slices = p.part_slices;
+  if (p.bm == 64)
+    return g.b_kn ? launch_mid_epi<64, true>(g, batch, p.parts, st)
+                  : launch_mid_epi<64, false>(g, batch, p.parts, st);
+  return g.b_kn ? launch_mid_epi<128, true>(g, batch, p.parts, st)
+                : launch_mid_epi<128, false>(g, batch, p.parts, st);
+}
+
 // 64 x 64 byte-tile transpose through LDS.
 __global__ __launch_bounds__(256) void transpose_u8_kernel(const uint8_t* src, uint8_t* dst,
                                                            int64_t R, int64_t C, int64_t lds,
@@ -867,7 +980,7 @@ static int gemm_run(const uint8_t* a8, const uint8_t* b8, int b_layout, const vo
                     void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                     int64_t ldc, float a_scale, float b_scale, const float* a_scale_dev,
                     const float* b_scale_dev, void* stream, const RowwiseBatch& rb = {},
-                    unsigned* item_counter = nullptr) {
+                    unsigned* item_counter = nullptr, size_t workspace_bytes = 0) {
   if (!a8 || !b8 || !c) {
     rp_set_error("gemm: null pointer");
     return RP_ERR_INVALID_ARGUMENT;
@@ -923,14 +1036,28 @@ static int gemm_run(const uint8_t* a8, const uint8_t* b8, int b_layout, const vo
   g.a_scale = a_scale; g.b_scale = b_scale; g.a_dev = a_scale_dev; g.b_dev = b_scale_dev;
   g.b_kn = kn ? 1 : 0;
   g.item_counter = item_counter;
-  // The large-tile kernel reads whole 64-byte K sub-slices and keeps tile
-  // offsets in 32 bits; from a (K, N) B it loads whole 16-byte N granules.
-  const bool big = K % kG2Sub == 0 && lda * (int64_t)kG2Tile < (int64_t)1 << 32 &&
-                   (kn ? (N % 16 == 0 && ldb % 16 == 0 && reinterpret_cast<uintptr_t>(b8) % 16 == 0 &&
-                          ldb * (int64_t)kG2K < (int64_t)1 << 32)
-                       : ldb * (int64_t)kG2Tile < (int64_t)1 << 32);
-  if (big) return launch_gemm256(g, rb.batch, static_cast<hipStream_t>(stream));
-  return launch_gemm<256, 128>(g, rb.batch, static_cast<hipStream_t>(stream));
+  // The direct-to-LDS kernels keep tile offsets in 32 bits and load whole
+  // 16-byte N granules from a (K, N) B; the 256 x 256 one reads whole
+  // 64-byte K sub-slices.
+  const bool direct = lda * (int64_t)kG2Tile < (int64_t)1 << 32 &&
+                      (kn ? (N % 16 == 0 && ldb % 16 == 0 &&
+                             reinterpret_cast<uintptr_t>(b8) % 16 == 0 &&
+                             ldb * (int64_t)kG2K < (int64_t)1 << 32)
+                          : ldb * (int64_t)kG2Tile < (int64_t)1 << 32);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (direct) {
+    const bool whole = K % kG2Sub == 0;
+    const bool split_ok = item_counter != nullptr && rb.row_scale == nullptr;
+    GemmPlan p = gemm_plan(M, N, K, rb.batch, whole, split_ok);
+    if (p.parts > 1 && workspace_bytes < gemm_workspace_bytes(M, N, p))
+      p = gemm_plan(M, N, K, rb.batch, whole, false);
+    if (p.parts > 1)
+      g.part = reinterpret_cast<float*>(reinterpret_cast<char*>(item_counter) +
+                                        RP_GEMM_BALANCED_WORKSPACE_BYTES);
+    if (p.bm != kG2Tile) return launch_gemm_mid(g, rb.batch, p, st);
+    return launch_gemm256(g, rb.batch, st);
+  }
+  return launch_gemm<256, 128>(g, rb.batch, st);
 }
 
 extern "C" int rp_fp8_gemm(const uint8_t* a8, const uint8_t* b8, int b_layout, void* c, int64_t M,
@@ -963,7 +1090,12 @@ extern "C" int rp_fp8_linear_balanced(const uint8_t* a8, const uint8_t* b8, int 
   }
   return gemm_run(a8, b8, b_layout, bias, c, M, N, K, lda, ldb, ldc, a_scale, b_scale,
                   a_scale_dev, b_scale_dev, stream, RowwiseBatch{},
-                  static_cast<unsigned*>(workspace));
+                  static_cast<unsigned*>(workspace), workspace_bytes);
+}
+
+extern "C" size_t rp_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return gemm_workspace_bytes(M, N, gemm_plan(M, N, K, 1, K % kG2Sub == 0, true));
 }
 
 extern "C" int rp_fp8_gemm_rowwise(const uint8_t* a8, const uint8_t* b8, int b_layout, void* c,

@@ -814,6 +814,11 @@ def transpose_fp8(x8: torch.Tensor) -> torch.Tensor:
     return out.view(x8.dtype) if x8.dtype != torch.uint8 else out
 
 
+@functools.lru_cache(maxsize=1024)
+def _linear_ws_bytes(M: int, N: int, K: int) -> int:
+    return int(C.lib().rp_fp8_linear_workspace_bytes(M, N, K))
+
+
 def fp8_gemm(a8: torch.Tensor, b8: torch.Tensor, a_scale: float | torch.Tensor,
              b_scale: float | torch.Tensor, *, b_transposed: bool = False,
              out: torch.Tensor | None = None, bias: torch.Tensor | None = None) -> torch.Tensor:
@@ -873,9 +878,9 @@ def fp8_gemm(a8: torch.Tensor, b8: torch.Tensor, a_scale: float | torch.Tensor,
             raise ValueError(f"bias must be a contiguous ({N},) tensor, got {tuple(bias.shape)}")
         if bias.data_ptr() % 8 != 0:          # the epilogue reads 4 bias values at a time
             bias = bias.clone()
-    # the balanced launch (tiles pooled across XCDs) needs a small workspace
-    # for its counter; the outputs are rp_fp8_gemm's / rp_fp8_linear's bits
-    ws = torch.empty(C.RP_GEMM_BALANCED_WORKSPACE_BYTES, dtype=torch.uint8, device=a8.device)
+    # the balanced launch needs a workspace for its tile counter and, where K
+    # is split (few rows), for the parts' fp32 sums
+    ws = torch.empty(_linear_ws_bytes(M, N, K), dtype=torch.uint8, device=a8.device)
     *sizes, stream = args
     C.check(C.lib().rp_fp8_linear_balanced(
         a8.data_ptr(), b8.data_ptr(), layout, bias.data_ptr() if bias is not None else None,
