@@ -50,32 +50,31 @@ struct PParams {
   float* rinv;             // [B*H*S] 1/sqrt(mean(x^2) + eps) of each row
   int64_t rows_per_group;  // S (per (b, h)) or B*H*S (per tensor)
   int64_t rpb;             // rows per block
-  int64_t nbg;             // blocks per group
+  int64_t nbg;             // partial maxima per group
+  // rotary launches (rope_body): rows [S] in nsr ranges of rpb, heads in nhc
+  // chunks of hc
+  int64_t nsr;
+  int hc, nhc;
 };
 
 // fp32 -> nearest-even bf16 value, held in fp32 (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ float bf16r(float f) { return (float)(__bf16)f; }
 
-// The normalised (and rotated) 8 elements [8c, 8c+8) of U rows at xrow[u]
-// (positions s[u], global rows row[u]), each exactly a bf16 value held in
-// fp32.  All D/8 threads of a row call this together (the sum of squares
-// and the half rotation cross threads).  The U rows go through each step
-// side by side, so their dependent chains (squares, butterfly, sqrt,
-// divide) overlap.  Without rotary tables the amax pass (STORE) writes
-// each row's r = 1/sqrt(mean(x^2) + eps) to p.rinv and the apply pass
-// (LOAD) reads it back instead of repeating the chain -- the same fp32
-// value, so both passes normalise identically.  With tables the apply pass
-// recomputes r: reading it back measured 4% slower there (0.595 against
-// 0.57 ms at (1, 32, 56320, 128)), while it saves 7% without them.
-// The rotary layout is a template parameter: with it as a runtime branch,
-// hipcc 7.2 merged the two layouts' code so that the interleaved path
-// skipped its own sign flips (rotated with stale registers).
 // Sum of the two lanes of a quad xor K apart (DPP quad_perm, no LDS trip).
 template <int K>
 __device__ __forceinline__ float add_quad_xor(float v) {
   static_assert(K == 1 || K == 2, "quad lanes");
   constexpr int sel = K == 1 ? 0xB1 : 0x4E;   // (1, 0, 3, 2) or (2, 3, 0, 1)
   const int r = __builtin_amdgcn_mov_dpp(__float_as_int(v), sel, 0xf, 0xf, false);
+  return v + __int_as_float(r);
+}
+
+// v + (v of lane ^ 4): lanes with bit 2 clear take the lane four up, the
+// others the lane four down (DPP row shifts, bank masks pick the quads).
+__device__ __forceinline__ float add_xor4(float v) {
+  const int x = __float_as_int(v);
+  int r = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0x5, false);   // row_shl:4, quads 0, 2
+  r = __builtin_amdgcn_update_dpp(r, x, 0x114, 0xf, 0xa, false);       // row_shr:4, quads 1, 3
   return v + __int_as_float(r);
 }
 
@@ -88,6 +87,11 @@ __device__ __forceinline__ float add_quad_xor(float v) {
 // The levels k >= TPR pair chunks of one thread; the others pair lanes.
 // With PMAX, pmax[u] also gets the two 16-bit maxima of |x| over the
 // thread's elements of row u, from the packed input bits.
+// The U rows go through each step side by side, so their dependent chains
+// (squares, butterfly, sqrt, divide) overlap.  The amax pass (STORE) writes
+// each row's r to p.rinv and the apply pass (LOAD) reads it back instead of
+// repeating the chain -- the same fp32 value, so both passes normalise
+// identically (7% of the prologue without tables).
 template <int D, int U, int EPT, bool LOAD, bool STORE, bool PMAX = false>
 __device__ __forceinline__ void load_norm(const PParams& p, const uint16_t* const (&xrow)[U],
                                           const int64_t (&row)[U], int c, float (&x)[U][EPT],
@@ -140,10 +144,11 @@ __device__ __forceinline__ void load_norm(const PParams& p, const uint16_t* cons
         ss[u][0] = add_row_ror<2>(ss[u][0]);
         ss[u][0] = add_row_ror<1>(ss[u][0]);
       }
-    } else if constexpr (TPR <= 4) {
+    } else if constexpr (TPR <= 8) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if constexpr (TPR == 4) ss[u][0] = add_quad_xor<2>(ss[u][0]);
+        if constexpr (TPR == 8) ss[u][0] = add_xor4(ss[u][0]);
+        if constexpr (TPR >= 4) ss[u][0] = add_quad_xor<2>(ss[u][0]);
         if constexpr (TPR >= 2) ss[u][0] = add_quad_xor<1>(ss[u][0]);
       }
     } else {
@@ -160,12 +165,12 @@ __device__ __forceinline__ void load_norm(const PParams& p, const uint16_t* cons
   }
 }
 
-template <int D, int ROPE, int U, int EPT, bool LOAD, bool STORE>
+// The normalised EPT elements of U rows, each exactly a bf16 value in fp32.
+template <int D, int U, int EPT, bool LOAD, bool STORE>
 __device__ __forceinline__ void prologue_rows(const PParams& p, const uint16_t* const (&xrow)[U],
-                                              const int64_t (&s)[U], const int64_t (&row)[U],
-                                              int c, float (&y)[U][EPT]) {
+                                              const int64_t (&row)[U], int c,
+                                              float (&y)[U][EPT]) {
 #pragma clang fp contract(off)
-  static_assert(ROPE == RP_ROPE_NONE || EPT == 8, "rotary rows: 8 elements per thread");
   constexpr int TPR = D / EPT;
   float x[U][EPT], r[U];
   load_norm<D, U, EPT, LOAD, STORE>(p, xrow, row, c, x, r);
@@ -189,39 +194,6 @@ __device__ __forceinline__ void prologue_rows(const PParams& p, const uint16_t* 
         }
     }
   }
-  if constexpr (ROPE == RP_ROPE_NONE) return;
-  else {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      float rot[8];
-      if constexpr (ROPE == RP_ROPE_HALF) {
-        // partner elements d +- D/2 live in thread c ^ (D/16)
-        const bool lo = c < D / 16;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float o = shfl_xor(y[u][i], D / 16);
-          rot[i] = lo ? -o : o;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-          rot[i] = -y[u][i + 1];
-          rot[i + 1] = y[u][i];
-        }
-      }
-      const float4* cp = reinterpret_cast<const float4*>(p.cosv + s[u] * D + 8 * c);
-      const float4* sp = reinterpret_cast<const float4*>(p.sinv + s[u] * D + 8 * c);
-      const float4 c0 = cp[0], c1 = cp[1], s0 = sp[0], s1 = sp[1];
-      const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-      const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float a = y[u][i] * cs[i];
-        const float b = rot[i] * sn[i];
-        y[u][i] = bf16r(a + b);
-      }
-    }
-  }
 }
 
 // (b, h, s) of a row, advanced without divisions.
@@ -236,27 +208,17 @@ struct PCursor {
   }
 };
 
-// Rows per thread and loop step: the rows of one step run side by side.
-// Measured at (1, 32, 56320, 128): without rotary tables 1/2/4 rows take
-// 0.296/0.246/0.251 ms; with tables (16 more fp32 values per row) one row
-// is fastest (0.57 ms, 0.63 with two).
-template <int ROPE>
-constexpr int kPRowsPerStep = ROPE == RP_ROPE_NONE ? 2 : 1;
-// Elements per thread and rows per step of the amax pass without rotary
-// tables.  Every thread of a row computes the row's inverse norm (IEEE sqrt
-// and divide, the butterfly), so fewer threads per row spread that over more
-// elements: 8 elements per thread took 14 VALU instructions per element.
-// Measured at C2 (1, 32, 56320, 128), Q/K/V in one call: 8/16/32 elements
-// per thread with two rows per step 0.628/0.626/0.622 ms, 32 with one row
-// 0.624 ms.
-template <int ROPE>
-constexpr int kAmaxEpt = ROPE == RP_ROPE_NONE ? 32 : 8;
-template <int ROPE>
-constexpr int kAmaxRows = kPRowsPerStep<ROPE>;
-
-// Whether the apply pass reads each row's inverse norm back from the amax pass.
-template <int ROPE>
-constexpr bool kStoreNorm = ROPE == RP_ROPE_NONE;
+// Rows per thread and loop step without rotary tables: the rows of one step
+// run side by side (1/2/4 rows took 0.296/0.246/0.251 ms at
+// (1, 32, 56320, 128)).
+constexpr int kPRowsPerStep = 2;
+// Elements per thread of the amax pass without rotary tables.  Every thread
+// of a row computes the row's inverse norm (IEEE sqrt and divide, the
+// butterfly), so fewer threads per row spread that over more elements: 8
+// elements per thread took 14 VALU instructions per element.  Measured at C2
+// (1, 32, 56320, 128), Q/K/V in one call: 8/16/32 elements per thread with
+// two rows per step 0.628/0.626/0.622 ms, 32 with one row 0.624 ms.
+constexpr int kAmaxEpt = 32;
 
 // Row iteration shared by both passes: block blk covers rows
 // [first, first + nrows) of group g; with TPR = D/EPT threads per row,
@@ -331,13 +293,13 @@ __device__ __forceinline__ void for_rows(const PParams& p, int64_t blk, F&& fn) 
   }
 }
 
-template <int D, int ROPE>
+template <int D>
 __device__ __forceinline__ void prologue_amax_body(const PParams& p, int64_t blk,
                                                    uint32_t* partial) {
-  constexpr int U = kAmaxRows<ROPE>;
-  constexpr int EPT = kAmaxEpt<ROPE>;
+  constexpr int U = kPRowsPerStep;
+  constexpr int EPT = kAmaxEpt;
   uint32_t m = 0;
-  if (ROPE == RP_ROPE_NONE && p.weight == nullptr) {
+  if (p.weight == nullptr) {
     // y = bf16(x * r) is only needed for its maximum, and for r >= 0 that is
     // bf16(max |x| * r): the product and the rounding are monotonic in |x|.
     // So each thread takes the maximum of its |x| from the packed input bits
@@ -353,7 +315,7 @@ __device__ __forceinline__ void prologue_amax_body(const PParams& p, int64_t blk
 #pragma clang fp contract(off)
       float x[U][EPT], rn[U];
       uint32_t pm[U];
-      load_norm<D, U, EPT, false, kStoreNorm<ROPE>, true>(p, xrow, r, c, x, rn, pm);
+      load_norm<D, U, EPT, false, true, true>(p, xrow, r, c, x, rn, pm);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         // the bf16 conversion of y in every other path (v_cvt_pk_bf16_f32)
@@ -368,10 +330,10 @@ __device__ __forceinline__ void prologue_amax_body(const PParams& p, int64_t blk
     });
   } else {
     for_rows<D, U, EPT>(p, blk, [&](const int64_t (&r)[U], const int64_t (&)[U],
-                                    const int64_t (&s)[U], const uint16_t* const (&xrow)[U],
+                                    const int64_t (&)[U], const uint16_t* const (&xrow)[U],
                                     const bool (&ok)[U], int c) {
       float y[U][EPT];
-      prologue_rows<D, ROPE, U, EPT, false, kStoreNorm<ROPE>>(p, xrow, s, r, c, y);
+      prologue_rows<D, U, EPT, false, true>(p, xrow, r, c, y);
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -392,11 +354,6 @@ __device__ __forceinline__ void prologue_amax_body(const PParams& p, int64_t blk
   }
 }
 
-template <int D, int ROPE>
-__global__ __launch_bounds__(kPThreads) void prologue_amax_kernel(PParams p, uint32_t* partial) {
-  prologue_amax_body<D, ROPE>(p, blockIdx.x, partial);
-}
-
 __global__ __launch_bounds__(kPThreads) void prologue_finalize_kernel(const uint32_t* partial,
                                                                       int64_t nbg,
                                                                       float* dequant) {
@@ -405,16 +362,16 @@ __global__ __launch_bounds__(kPThreads) void prologue_finalize_kernel(const uint
   if (threadIdx.x == 0) dequant[g] = dequant_from_amax_bits(r);
 }
 
-template <int D, int ROPE>
+template <int D>
 __device__ __forceinline__ void prologue_quant_body(const PParams& p, int64_t blk,
                                                     const float* dequant, int per_bh,
                                                     uint8_t* codes) {
-  constexpr int U = kPRowsPerStep<ROPE>;
+  constexpr int U = kPRowsPerStep;
   for_rows<D, U, 8>(p, blk, [&](const int64_t (&r)[U], const int64_t (&bh)[U],
-                                const int64_t (&s)[U], const uint16_t* const (&xrow)[U],
+                                const int64_t (&)[U], const uint16_t* const (&xrow)[U],
                                 const bool (&ok)[U], int c) {
     float y[U][8];
-    prologue_rows<D, ROPE, U, 8, kStoreNorm<ROPE>, false>(p, xrow, s, r, c, y);
+    prologue_rows<D, U, 8, true, false>(p, xrow, r, c, y);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (!ok[u]) continue;
@@ -430,11 +387,234 @@ __device__ __forceinline__ void prologue_quant_body(const PParams& p, int64_t bl
   });
 }
 
+// ---- rows with rotary tables
+//
+// A block takes a range of rows (positions s) of several heads: a thread
+// keeps its row's cos and sin (16 elements each) in registers and applies
+// them to the heads of the block's chunk one after another.  With a head per
+// block, as the plain rows run, every head reads the whole fp32 (S, D)
+// tables again -- 64 bytes of L2 / MALL traffic per 16 bytes of input, 3.7 GB
+// per pass over Q and K at (1, 32, 56320, 128), which was the pass's time;
+// eight heads per block leave 8 bytes per 16.  Row ranges that lie eight
+// apart in block order share an XCD's L2, so the chunks of one range find
+// its tables there.
+//
+// D/16 threads share a row; thread c holds 16-byte chunks c and c + D/16,
+// that is elements d and their half-rotation partners d + D/2: neither
+// layout crosses threads, and the row's inverse norm (butterfly, IEEE sqrt
+// and divide) is repeated by half as many threads as one chunk each would.
+// The rotary layout is a template parameter: with it as a runtime branch,
+// hipcc 7.2 merged the two layouts' code so that the interleaved path
+// skipped its own sign flips (rotated with stale registers).
+//
+// Bound by HBM and VALU alike (~14-18 instructions per element and pass).
+// Q, K and V of (1, 32, 56320, 128) in one call, weights and half-rotation
+// tables: 1.46 ms (amax 0.66-0.68, apply 0.77) with one head per block and one
+// chunk per thread, 0.674 ms here; 4 or 16 heads per block 0.692 / 0.675 ms.
+constexpr int kRopeMaxHeads = 16;   // LDS words for a block's heads
+constexpr int kRopeHeads = 8;       // heads per block
+// Fewer heads per block below this many blocks (per tensor): at
+// (1, 40, 16384, 128) 1024 and 256 take 0.264 and 0.267 ms, 3000 0.284 ms.
+constexpr int64_t kRopeMinBlocks = 1024;
+
+// two fp32 -> their nearest-even bf16 values as fp32 (one v_cvt_pk_bf16_f32)
+// and the packed pair
+__device__ __forceinline__ uint32_t bf16r2(float& a, float& b) {
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
+  a = bf16_to_f32(w & 0xffffu);
+  b = bf16_to_f32(w >> 16);
+  return w;
+}
+
+// Normalised and rotated elements of one row, in place: x[0..8) is chunk c
+// and x[8..16) chunk c + D/16; `w` the weight's bits of both chunks (pairs),
+// cs and sn their cos and sin.  Returns the packed |y| pair maxima.
+template <int ROPE>
+__device__ __forceinline__ uint32_t rope_row(float (&x)[16], float r, bool has_w,
+                                             const uint32_t (&w)[8], const float (&cs)[16],
+                                             const float (&sn)[16]) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) {
+    x[i] = x[i] * r;
+    x[i + 1] = x[i + 1] * r;
+    bf16r2(x[i], x[i + 1]);
+  }
+  if (has_w) {
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+      x[i] = x[i] * bf16_to_f32(w[i / 2] & 0xffffu);
+      x[i + 1] = x[i + 1] * bf16_to_f32(w[i / 2] >> 16);
+      bf16r2(x[i], x[i + 1]);
+    }
+  }
+  float y[16];
+  if constexpr (ROPE == RP_ROPE_HALF) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // rot = -(upper) for the lower half: a + (-u * s) == a - u * s exactly
+      const float l = x[i], u = x[i + 8];
+      const float al = l * cs[i], bl = u * sn[i];
+      const float au = u * cs[i + 8], bu = l * sn[i + 8];
+      y[i] = al - bl;
+      y[i + 8] = au + bu;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+      const float e = x[i], o = x[i + 1];
+      const float ae = e * cs[i], be = o * sn[i];
+      const float ao = o * cs[i + 1], bo = e * sn[i + 1];
+      y[i] = ae - be;
+      y[i + 1] = ao + bo;
+    }
+  }
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) {
+    const uint32_t pk = bf16r2(y[i], y[i + 1]);
+    m = pk_max_u16(m, pk & 0x7fff7fffu);
+    x[i] = y[i];
+    x[i + 1] = y[i + 1];
+  }
+  return m;
+}
+
+// Block b of one tensor.  APPLY: codes under the given scales; else the
+// partial maxima, one per (head, row range).
+template <int D, int ROPE, bool APPLY>
+__device__ __forceinline__ void rope_body(const PParams& p, int64_t b, uint32_t* partial,
+                                          const float* dequant, int per_bh, uint8_t* codes) {
+  constexpr int TPR = D / 16;                    // threads per row
+  constexpr int RPI = kPThreads / TPR;           // rows per iteration
+  constexpr int RPB = (int)(kPElemsPerBlock / D);
+  static_assert(RPB % RPI == 0, "whole iterations");
+  constexpr int U = 2;                           // heads side by side
+  __shared__ uint32_t s_max[kRopeMaxHeads];
+  __shared__ float s_qm[kRopeMaxHeads];
+  const int64_t q = b >> 3;
+  const int64_t hcI = q % p.nhc;
+  const int64_t sr = (q / p.nhc) * 8 + (b & 7);
+  if (sr >= p.nsr) return;
+  const int bh0 = (int)hcI * p.hc;
+  const int nh = min(p.hc, (int)(p.B * p.H) - bh0);
+  if ((int)threadIdx.x < nh) {
+    if constexpr (APPLY) s_qm[threadIdx.x] = 1.0f / dequant[per_bh ? bh0 + threadIdx.x : 0];
+    else s_max[threadIdx.x] = 0;
+  }
+  __syncthreads();
+  const int c = threadIdx.x % TPR;
+  uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  const bool has_w = p.weight != nullptr;
+  if (has_w) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const uint4 v = *reinterpret_cast<const uint4*>(p.weight + 8 * (c + TPR * m));
+      w[4 * m] = v.x; w[4 * m + 1] = v.y; w[4 * m + 2] = v.z; w[4 * m + 3] = v.w;
+    }
+  }
+#pragma unroll 1
+  for (int it = 0; it < RPB / RPI; ++it) {
+    const int64_t s_own = sr * RPB + it * RPI + threadIdx.x / TPR;
+    if (sr * RPB + it * RPI >= p.S) break;
+    const bool ok = s_own < p.S;
+    const int64_t s = ok ? s_own : p.S - 1;      // read, never used
+    float cs[16], sn[16];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const f32x4* cp = reinterpret_cast<const f32x4*>(p.cosv + s * D + 8 * (c + TPR * m));
+      const f32x4* sp = reinterpret_cast<const f32x4*>(p.sinv + s * D + 8 * (c + TPR * m));
+      const f32x4 c0 = cp[0], c1 = cp[1], s0 = sp[0], s1 = sp[1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        cs[8 * m + i] = c0[i]; cs[8 * m + 4 + i] = c1[i];
+        sn[8 * m + i] = s0[i]; sn[8 * m + 4 + i] = s1[i];
+      }
+    }
+#pragma unroll 1
+    for (int h = 0; h < nh; h += U) {
+      float x[U][16], r[U];
+      const uint16_t* xrow[U];
+      int64_t row[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // an odd chunk's last step repeats its head
+        const int bh = bh0 + min(h + u, nh - 1);
+        const int bb = bh / (int)p.H;
+        xrow[u] = p.x + bb * p.sb + (bh - bb * (int)p.H) * p.sh + s * p.ss;
+        row[u] = (int64_t)bh * p.S + s;
+      }
+      load_norm<D, U, 16, APPLY, !APPLY>(p, xrow, row, c, x, r);
+      uint32_t m[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) m[u] = rope_row<ROPE>(x[u], r[u], has_w, w, cs, sn);
+      if constexpr (!APPLY) {
+        // both heads' maxima through one reduction, a 16-bit half each
+        uint32_t v = 0;
+        if (ok) v = umax32(m[0] & 0xffffu, m[0] >> 16) | (umax32(m[1] & 0xffffu, m[1] >> 16) << 16);
+#pragma unroll
+        for (int o = 1; o <= 32; o <<= 1) v = pk_max_u16(v, (uint32_t)shfl_xor((int)v, o));
+        if ((threadIdx.x & (kWave - 1)) == 0) {
+          atomicMax(&s_max[h], v & 0xffffu);
+          atomicMax(&s_max[min(h + 1, nh - 1)], v >> 16);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float qm = s_qm[min(h + u, nh - 1)];
+          // |y * qm| <= 426.7 under the row's own scale: the clamp of the
+          // plain conversion never binds for a bf16 y (and a NaN or infinite
+          // maximum makes every code of the group NaN or 0 either way)
+          uint32_t o[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = pack4_e4m3(x[u][4 * i] * qm, x[u][4 * i + 1] * qm, x[u][4 * i + 2] * qm,
+                              x[u][4 * i + 3] * qm);
+          // chunk c is o[0..1], chunk c + D/16 o[2..3]: neighbours (c even,
+          // c + 1) trade, so that the even lane holds chunks c, c + 1 and the
+          // odd lane their upper partners -- 16 bytes each, whole lines per row
+          const bool odd = c & 1;
+          const uint32_t give0 = odd ? o[0] : o[2], give1 = odd ? o[1] : o[3];
+          const uint32_t got0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)give0, 0xB1, 0xf, 0xf, false);
+          const uint32_t got1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)give1, 0xB1, 0xf, 0xf, false);
+          const u32x4 v = odd ? u32x4{got0, got1, o[2], o[3]} : u32x4{o[0], o[1], got0, got1};
+          if (ok && h + u < nh)
+            __builtin_nontemporal_store(
+                v, reinterpret_cast<u32x4*>(codes + row[u] * D + 8 * (odd ? c - 1 + TPR : c)));
+        }
+      }
+    }
+  }
+  if constexpr (!APPLY) {
+    __syncthreads();
+    if ((int)threadIdx.x < nh) partial[(bh0 + threadIdx.x) * p.nsr + sr] = s_max[threadIdx.x];
+  }
+}
+
+// One block of a tensor's pass, with or without tables.
+template <int D, int ROPE>
+__device__ __forceinline__ void amax_block(const PParams& p, int64_t blk, uint32_t* partial) {
+  if constexpr (ROPE == RP_ROPE_NONE) prologue_amax_body<D>(p, blk, partial);
+  else rope_body<D, ROPE, false>(p, blk, partial, nullptr, 0, nullptr);
+}
+template <int D, int ROPE>
+__device__ __forceinline__ void quant_block(const PParams& p, int64_t blk, const float* dequant,
+                                            int per_bh, uint8_t* codes) {
+  if constexpr (ROPE == RP_ROPE_NONE) prologue_quant_body<D>(p, blk, dequant, per_bh, codes);
+  else rope_body<D, ROPE, true>(p, blk, nullptr, dequant, per_bh, codes);
+}
+
+template <int D, int ROPE>
+__global__ __launch_bounds__(kPThreads) void prologue_amax_kernel(PParams p, uint32_t* partial) {
+  amax_block<D, ROPE>(p, blockIdx.x, partial);
+}
 template <int D, int ROPE>
 __global__ __launch_bounds__(kPThreads) void prologue_quant_kernel(PParams p,
                                                                    const float* dequant,
                                                                    int per_bh, uint8_t* codes) {
-  prologue_quant_body<D, ROPE>(p, blockIdx.x, dequant, per_bh, codes);
+  quant_block<D, ROPE>(p, blockIdx.x, dequant, per_bh, codes);
 }
 
 // ---- Q and K through the prologue, V through the plain quantizer, together:
@@ -464,9 +644,9 @@ __global__ __launch_bounds__(kPThreads) void qkv_norm_amax_kernel(NormQKV a) {
   const int t = blockIdx.x % 3;
   const int64_t b = blockIdx.x / 3;
   if (t == 0) {
-    if (b < a.nq) prologue_amax_body<D, ROPE>(a.q, b, a.pq);
+    if (b < a.nq) amax_block<D, ROPE>(a.q, b, a.pq);
   } else if (t == 1) {
-    if (b < a.nk) prologue_amax_body<D, ROPE>(a.k, b, a.pk);
+    if (b < a.nk) amax_block<D, ROPE>(a.k, b, a.pk);
   } else if (b < a.nv) {
     if (a.vflat) amax_flat_body(b, a.v.x, a.vgsize, a.v.nbg, a.pv);
     else amax_partial_body(b, a.v, a.pv);
@@ -486,9 +666,9 @@ __global__ __launch_bounds__(kPThreads) void qkv_norm_apply_kernel(NormQKV a) {
   const int t = blockIdx.x % 3;
   const int64_t b = blockIdx.x / 3;
   if (t == 0) {
-    if (b < a.nq) prologue_quant_body<D, ROPE>(a.q, b, a.dequant, a.per_bh, a.q8);
+    if (b < a.nq) quant_block<D, ROPE>(a.q, b, a.dequant, a.per_bh, a.q8);
   } else if (t == 1) {
-    if (b < a.nk) prologue_quant_body<D, ROPE>(a.k, b, a.dequant + a.ngroups, a.per_bh, a.k8);
+    if (b < a.nk) quant_block<D, ROPE>(a.k, b, a.dequant + a.ngroups, a.per_bh, a.k8);
   } else if (b < a.nvt) {
     // 128 rows of one head of V: its D/64 column tiles one after the other
     const int64_t bh = b / a.vt_tiles;
@@ -511,10 +691,15 @@ int launch_check(const char* what) {
   return RP_OK;
 }
 
+// Blocks of one tensor's pass.
+inline int64_t prologue_blocks(const PParams& p, int64_t ngroups) {
+  return p.cosv != nullptr ? (p.nsr + 7) / 8 * 8 * p.nhc : ngroups * p.nbg;
+}
+
 template <int D, int ROPE>
 int run_prologue(const PParams& p, int64_t ngroups, float* dequant, uint8_t* codes, int per_bh,
                  uint32_t* partial, hipStream_t st) {
-  const unsigned blocks = (unsigned)(ngroups * p.nbg);
+  const unsigned blocks = (unsigned)prologue_blocks(p, ngroups);
   hipLaunchKernelGGL((prologue_amax_kernel<D, ROPE>), dim3(blocks), dim3(kPThreads), 0, st, p,
                      partial);
   int rc = launch_check("rmsnorm_quantize(amax)");
@@ -552,10 +737,9 @@ struct PSizes {
 bool prologue_sizes(int64_t B, int64_t H, int64_t S, int64_t D, int granularity, PSizes* out) {
   if (B <= 0 || H <= 0 || S <= 0 || (D != 64 && D != 128)) return false;
   if (granularity != RP_SCALE_PER_BH && granularity != RP_SCALE_PER_TENSOR) return false;
-  const int64_t ngroups = granularity == RP_SCALE_PER_BH ? B * H : 1;
-  const int64_t rows = B * H * S / ngroups;
   const int64_t rpb = kPElemsPerBlock / D;
-  out->partials = (size_t)(ngroups * ((rows + rpb - 1) / rpb)) * sizeof(uint32_t);
+  // one per head and row range (the most either kind of row writes)
+  out->partials = (size_t)(B * H * ((S + rpb - 1) / rpb)) * sizeof(uint32_t);
   out->rinv = (size_t)(B * H * S) * sizeof(float);
   return true;
 }
@@ -617,7 +801,16 @@ int make_pparams(const char* who, const void* x, int64_t B, int64_t H, int64_t S
   p.rows_per_group = B * H * S / ngroups;
   p.rpb = kPElemsPerBlock / D;
   p.nbg = (p.rows_per_group + p.rpb - 1) / p.rpb;
-  if (3 * ngroups * p.nbg > 0x7fffffffLL) {
+  if (p.cosv != nullptr) {
+    p.nsr = (S + p.rpb - 1) / p.rpb;
+    p.nbg = p.nsr * (B * H / ngroups);
+    // heads per block: the more, the fewer reads of the tables, as long as
+    // the blocks cover the GPU several times over
+    p.hc = kRopeHeads;
+    while (p.hc > 2 && p.nsr * ((B * H + p.hc - 1) / p.hc) < kRopeMinBlocks) p.hc /= 2;
+    p.nhc = (int)((B * H + p.hc - 1) / p.hc);
+  }
+  if (B * H > 0x7fffffffLL || 3 * max(ngroups * p.nbg, prologue_blocks(p, ngroups)) > 0x7fffffffLL) {
     rp_set_error("%s: grid too large", who);
     return RP_ERR_UNSUPPORTED;
   }
@@ -746,8 +939,8 @@ extern "C" int rp_fp8_rmsnorm_scale_quantize_qkv(
   a.vflat = pv.flat;
   a.per_bh = granularity == RP_SCALE_PER_BH;
   a.vgsize = pv.gsize;
-  a.nq = ngroups * a.q.nbg;
-  a.nk = ngroups * a.k.nbg;
+  a.nq = prologue_blocks(a.q, ngroups);
+  a.nk = prologue_blocks(a.k, ngroups);
   a.nv = pv.p.ngroups * pv.p.nbg;
   a.vt_tiles = ldv / 128;
   a.nvt = B * H * a.vt_tiles;
@@ -760,9 +953,9 @@ extern "C" int rp_fp8_rmsnorm_scale_quantize_qkv(
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   size_t off = 0;
   a.pq = reinterpret_cast<uint32_t*>(ws + off);
-  off += align256((size_t)a.nq * sizeof(uint32_t));
+  off += align256((size_t)(ngroups * a.q.nbg) * sizeof(uint32_t));
   a.pk = reinterpret_cast<uint32_t*>(ws + off);
-  off += align256((size_t)a.nk * sizeof(uint32_t));
+  off += align256((size_t)(ngroups * a.k.nbg) * sizeof(uint32_t));
   a.pv = reinterpret_cast<uint32_t*>(ws + off);
   off += align256(pv.ws_bytes);
   a.q.rinv = reinterpret_cast<float*>(ws + off);

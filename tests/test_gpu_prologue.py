@@ -207,3 +207,27 @@ def test_unit_weight_is_the_identity_on_extremes(gpu: torch.device, gran: str) -
         dq_b, c_b = ops.rmsnorm_scale_quantize(x, ones, eps, None, "half", gran)
         assert torch.equal(dq_a.view(torch.int32), dq_b.view(torch.int32)), eps
         assert torch.equal(c_a.view(torch.uint8), c_b.view(torch.uint8)), eps
+
+
+@pytest.mark.parametrize("rope,gran", [("half", "bh"), ("interleaved", "tensor")])
+def test_rotary_head_chunks_equal_single_heads(gpu: torch.device, rope: str, gran: str) -> None:
+    """Large rotary calls run several heads per block (eight here, the ninth
+    head alone in the last chunk, a ragged last row range): every head's codes
+    equal those of a call on that head alone, which runs one chunk of one
+    head, under the same scale."""
+    B, H, S, D = 1, 9, 66013, 128
+    g = torch.Generator(device=gpu).manual_seed(3)
+    x = (torch.randn((B, S, H, D), generator=g, device=gpu) * 2).to(torch.bfloat16)
+    x = x.permute(0, 2, 1, 3)
+    w = _x(5, (D,), 0.8).to(gpu)
+    t = tuple(torch.from_numpy(a).to(gpu) for a in _tables(S, D))
+    dq, codes = ops.rmsnorm_scale_quantize(x, w, 1e-6, t, rope, gran)
+    one = [ops.rmsnorm_scale_quantize(x[:, h:h + 1], w, 1e-6, t, rope, "bh") for h in range(H)]
+    if gran == "bh":
+        assert torch.equal(dq, torch.cat([d for d, _ in one]))
+        for h in range(H):
+            assert torch.equal(codes[:, h].view(torch.uint8), one[h][1][:, 0].view(torch.uint8))
+    else:
+        top = max(range(H), key=lambda h: float(one[h][0]))
+        assert float(dq) == float(one[top][0])
+        assert torch.equal(codes[:, top].view(torch.uint8), one[top][1][:, 0].view(torch.uint8))
