@@ -121,6 +121,7 @@ struct AttnArgs {
   unsigned* item_counter;
   int n_grid;
   int pool_r;   // unsplit items per XCD share that go to the pool
+  int longest_first;   // causal blocks in descending order of their key tiles
 };
 
 // Output kinds of the attention kernel.
@@ -574,18 +575,46 @@ void attn_fwd_kernel(AttnArgs a) {
   }
   // the two halves of a split query block are neighbours: same XCD, same
   // K tiles in its L2
-  const int half = DV < DK ? L2 & 1 : 0;
+  int half = DV < DK ? L2 & 1 : 0;
   const int L = DV < DK ? L2 >> 1 : L2;
-  const int dv_off = half * DV;  // first O column / V^T row of this workgroup
   // the items' query blocks [first_qb, first_qb + nqb) and key splits
   const int first_qb = MIXED && !part ? 0 : a.qb_begin;
   const int nqb = MIXED ? (part ? a.n_qblocks - a.qb_begin : a.qb_begin) : a.n_qblocks;
   const int nsplit = MIXED && !part ? 1 : a.kv_splits;
   const int per_bh = MULTI ? a.wg_per_bh : nqb * nsplit;
-  const int bh = L / per_bh;
-  const int qb = MULTI ? (L - bh * per_bh) * a.qb_per_wg
-                       : (L - bh * per_bh) / nsplit + first_qb;
-  const int split = MULTI ? 0 : L - bh * per_bh - (qb - first_qb) * nsplit;
+  int bh = L / per_bh;
+  int qb = MULTI ? (L - bh * per_bh) * a.qb_per_wg
+                 : (L - bh * per_bh) / nsplit + first_qb;
+  if constexpr (WINDOW && OUT != kOutSplit) {
+    if (a.longest_first) {
+      // Causal blocks run longest first: block qb has about 2 qb + 2 key
+      // tiles, and a launch in ascending order ends with its longest blocks
+      // alone on a few CUs (32 heads x 4096: 136 us, against 146 without the
+      // mask and twice its work).  Dispatch hands out workgroups in order, so
+      // the blocks of every head of a chunk go out in descending qb, the
+      // heads side by side: longer blocks first and each CU's second block
+      // the shorter the longer its first was.  Chunks of 32 heads keep the
+      // K/V streams of an XCD (w % 8: heads 8 apart) few enough to share its
+      // L2.  32 x 4096 keys and queries: 136 -> 100 us; 32 x 8192: 370 -> 336;
+      // 32 x 16384: 1209 -> 1181.  A grid of one round keeps the plain order,
+      // whose heads stay on one XCD whatever their number (12 heads x 3000:
+      // 2.4% slower in this one).
+      const int items = DV < DK ? a.n_work >> 1 : a.n_work;
+      // the halves of a split block stay neighbours on their XCD where the
+      // blocks divide over the XCDs
+      const bool even = DV < DK && (items & 7) == 0;
+      const int it = DV == DK ? w : even ? (k_x >> 1) * 8 + xcd : w >> 1;
+      if (DV < DK) half = even ? k_x & 1 : w & 1;
+      const int per_chunk = 32 * a.n_qblocks;
+      const int chunk = it / per_chunk, r = it - chunk * per_chunk;
+      const int nh = min(32, a.B * a.H - 32 * chunk);
+      bh = 32 * chunk + r % nh;
+      qb = a.n_qblocks - 1 - r / nh;
+    }
+  }
+  const int dv_off = half * DV;  // first O column / V^T row of this workgroup
+  const int split = MULTI || (WINDOW && OUT != kOutSplit)
+                        ? 0 : L - bh * per_bh - (qb - first_qb) * nsplit;
   const int nblk = MULTI ? min(a.qb_per_wg, a.n_qblocks - qb) : 1;  // query blocks
   const int b = bh / a.H, h = bh - b * a.H;
 
@@ -898,7 +927,9 @@ void attn_fwd_kernel(AttnArgs a) {
       // the max over the tile's visible keys.  It is not when a shifted tile
       // opens a key split (its repeats belong to the previous split), nor
       // under a window mask: such a tile takes its max after the phase, from
-      // the masked scores.
+      // the masked scores.  (Taking it between the MFMAs there too, and again
+      // from the masked scores where the mask cuts the tile, was 2% slower at
+      // 16 causal heads x 16384: 654 against 641 us per call.)
       float mh[8];
       mfma_phase<DK, DV, LOADS, !WINDOW>(kl, vl, qop, pop, s, acc, alpha, mh, tl, nxt);
       // the next block's Q, after the tile loads (so a counted wait can leave
@@ -1294,6 +1325,7 @@ int launch_attn(const AttnArgs& base, int out_dtype, hipStream_t st) {
     return RP_ERR_UNSUPPORTED;
   }
   a.n_grid = (int)grid;
+  a.longest_first = a.mask == RP_MASK_CAUSAL && a.kv_splits == 1 && work > kCUs;
   if (a.kv_splits == 1) {
     if (kind == kOutF32)
       launch_fwd<D, kOutF32>(a, st);
