@@ -1244,12 +1244,20 @@ inline TailPlan tail_plan(int B, int H, int Sq, int Skv, int D, int mask, int cu
   // the unsplit workgroups spread evenly over the 8 XCDs
   if (m == nq || m == 0 || (per_block * m) % 8 != 0) return t;
   const int64_t tail = per_block * (nq - m);
-  auto rounds = [&](int64_t w, int s) { return (double)((w + cus - 1) / cus) / s; };
-  double best = rounds(tail, 1);
+  // In key tiles (~2 us): rounds of workgroups of n_kb / sp tiles and the
+  // fixed cost each, and for a split the merge launch (~5 us) and the parts,
+  // 128 KiB each, written and read at ~4 TB/s.  (Without the fixed cost and
+  // the parts' bytes the plan split 224 of (1, 32, 14080, 14080, 128)'s 1760
+  // workgroups eight ways: the call took 1.86 ms, 1.75 unsplit.)
+  auto cost_of = [&](int sp) {
+    const double parts = (double)tail * sp;
+    return (double)((tail * sp + cus - 1) / cus) * ((double)n_kb / sp + (double)kFixedTiles) +
+           (sp > 1 ? 2.5 + parts * 0.033 : 0.0);
+  };
+  double best = cost_of(1);
   int best_s = 1;
   for (int sp = 2; sp <= 8 && 2 * sp <= n_kb; sp *= 2) {
-    // ~0.05 of a round for the partial results and the merge
-    const double cost = rounds(tail * sp, sp) + 0.05;
+    const double cost = cost_of(sp);
     if (cost < best) {
       best = cost;
       best_s = sp;
