@@ -176,6 +176,132 @@ __global__ __launch_bounds__(kQThreads) void apply_fold_multi_kernel(QJobs3 jobs
   }
 }
 
+// Calls whose groups have at most 65536 elements: a workgroup of 1024 threads
+// per (tensor, group) reads the group once into registers (NV 16-byte vectors
+// per thread), reduces its maximum, computes its scale and quantizes what it
+// holds -- one launch, no partial maxima, no second read.  V^T's groups are
+// held as the 128 x 64 tiles of the transposing apply, four at a time.
+// The host's launches bound calls this small, so the launch saved is what
+// counts: attention over (1, 8, 1024, 64) takes 23.1 us per call against
+// 26.9 with the amax and folded apply launches, (2, 40, 512, 128) 30.8
+// against 38.0.  On the GPU one CU per group is just level with those two at
+// 65536 elements (10.3 us against 3.7 + 5.7 and a gap: ~6 VALU instructions
+// per element on one CU) and behind past it (131072: 17.1 against 3.6 + 5.5).
+constexpr int kGroupThreads = 1024;
+constexpr int kGroupVecs = 8;        // 16-byte vectors per thread: 65536 elements per group
+
+template <int DT>
+__global__ __launch_bounds__(kGroupThreads) void quant_group_kernel(QJobs3 jobs, QParams vt,
+                                                                    int64_t ld, int vt_stiles,
+                                                                    int vt_dtiles,
+                                                                    int vt_tiles_per_group,
+                                                                    uint8_t* vt8) {
+  constexpr int NV = kGroupVecs;
+  constexpr int SUB = kGroupThreads / kQThreads;   // V^T tiles side by side
+  __shared__ __attribute__((aligned(16))) uint8_t tile[SUB * kTileBytes];
+  __shared__ uint32_t wmax[kGroupThreads / kWave];
+  const QJob& jb = job_of(jobs);
+  const int64_t g = blockIdx.x;
+  const bool is_v = blockIdx.y == 2;
+  const int sub = threadIdx.x / kQThreads, t = threadIdx.x % kQThreads;
+  u32x4 v[NV];
+  if (!is_v) {
+    const int n8 = (int)(jb.gsize / 8);
+    const int mask = (1 << jb.p.vpr_log2) - 1;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = threadIdx.x + i * kGroupThreads;
+      v[i] = u32x4{0u, 0u, 0u, 0u};
+      if (idx >= n8) continue;
+      const uint16_t* src;
+      if (jb.flat) {
+        src = jb.p.x + g * jb.gsize + (int64_t)idx * 8;
+      } else {
+        // row of the (B, H, S, D) view: rows of a group of at most 65536
+        // elements, and their head, in 32 bits
+        const uint32_t r = (uint32_t)(idx >> jb.p.vpr_log2);
+        const uint32_t dbh = r / (uint32_t)jb.p.S, s = r - dbh * (uint32_t)jb.p.S;
+        const uint32_t bh = (uint32_t)(g * (jb.p.rows_per_group / jb.p.S)) + dbh;
+        const uint32_t b = bh / (uint32_t)jb.p.H, h = bh - b * (uint32_t)jb.p.H;
+        src = jb.p.x + b * jb.p.sb + h * jb.p.sh + s * jb.p.ss + (idx & mask) * 8;
+      }
+      v[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
+    }
+  } else {
+    // thread t of tile 4k + sub of the group: rows 4q + i, column chunk c
+    const int q = t >> 3, c = t & 7;
+#pragma unroll
+    for (int k = 0; k < NV / 4; ++k) {
+      const int tl = SUB * k + sub;
+      const int64_t gt = g * vt_tiles_per_group + tl;
+      const int64_t sb = gt % vt_stiles, rest = gt / vt_stiles;
+      const int64_t db = rest % vt_dtiles, bh = rest / vt_dtiles;
+      const int dcols = (int)min((int64_t)64, vt.D - db * 64);
+      const uint16_t* base = vt.x + (bh / vt.H) * vt.sb + (bh % vt.H) * vt.sh + db * 64 + c * 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t s = sb * 128 + 4 * q + i;
+        v[4 * k + i] = u32x4{0u, 0u, 0u, 0u};
+        if (tl < vt_tiles_per_group && s < vt.S && c * 8 < dcols)
+          v[4 * k + i] = __builtin_nontemporal_load(
+              reinterpret_cast<const u32x4*>(base + s * vt.ss));
+      }
+    }
+  }
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = pk_max_u16(m, v[i][e] & 0x7fff7fffu);
+  m = umax32(m & 0xffffu, m >> 16);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) m = umax32(m, (uint32_t)shfl_xor((int)m, o));
+  if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x / kWave] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kGroupThreads / kWave; ++w) m = umax32(m, wmax[w]);
+  const float dq = dequant_from_amax<DT>(m);
+  const float qm = 1.0f / dq;
+  if (threadIdx.x == 0) jb.dequant[g] = dq;
+  if (!is_v) {
+    const int n8 = (int)(jb.gsize / 8);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = threadIdx.x + i * kGroupThreads;
+      if (idx < n8)
+        __builtin_nontemporal_store(
+            u32x2{quant4<DT>(v[i][0], v[i][1], qm), quant4<DT>(v[i][2], v[i][3], qm)},
+            reinterpret_cast<u32x2*>(jb.codes + g * jb.gsize + (int64_t)idx * 8));
+    }
+    return;
+  }
+  uint8_t* const own = tile + sub * kTileBytes;
+#pragma unroll
+  for (int k = 0; k < NV / 4; ++k) {
+    if (SUB * k >= vt_tiles_per_group) break;      // uniform
+    const int tl = SUB * k + sub;
+    uint32_t w[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      w[i][0] = quant4<DT>(v[4 * k + i][0], v[4 * k + i][1], qm);
+      w[i][1] = quant4<DT>(v[4 * k + i][2], v[4 * k + i][3], qm);
+    }
+    // rows past S and columns past D hold zeros, whose codes are 0 under any
+    // finite scale; under a NaN scale they would not be (V^T's padding must)
+    const int q = t >> 3, c = t & 7;
+    const int64_t gt = g * vt_tiles_per_group + tl;
+    const int64_t sb = gt % vt_stiles, rest = gt / vt_stiles;
+    const int64_t db = rest % vt_dtiles, bh = rest / vt_dtiles;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (sb * 128 + 4 * q + i >= vt.S || c * 8 >= vt.D - db * 64) w[i][0] = w[i][1] = 0u;
+    if (k > 0) __syncthreads();   // every thread has read the previous tiles
+    apply_t_put(w, own, t);
+    __syncthreads();
+    if (tl < vt_tiles_per_group) apply_t_out(vt, vt8, ld, sb, db, bh, own, t);
+  }
+}
+
 __global__ void selftest_e4m3_kernel(const float* x, uint8_t* out, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -418,11 +544,26 @@ static int qkv_launch(const Plan& pq, const Plan& pk, const Plan& pv, const void
     return RP_ERR_UNSUPPORTED;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t vt_stiles = ldv / 128, vt_dtiles = (D + 63) / 64;
+  const int64_t vt_blocks = vt_stiles * vt_dtiles * B * H;
+  // groups that fit one workgroup's registers: one launch
+  const int64_t gmax = max(pq.gsize, pk.gsize), gtiles = vt_blocks / ng;
+  if (q8 != nullptr && gmax <= (int64_t)kGroupThreads * 8 * kGroupVecs && gtiles <= kGroupVecs) {
+    QParams vt{};
+    vt.x = static_cast<const uint16_t*>(v);
+    vt.B = B; vt.H = H; vt.S = Skv; vt.D = D; vt.sb = vsb; vt.sh = vsh; vt.ss = vss;
+    const dim3 grid((unsigned)ng, 3), block(kGroupThreads);
+    if (x_dtype == RP_DTYPE_F16)
+      hipLaunchKernelGGL(quant_group_kernel<kInF16>, grid, block, 0, st, jobs, vt, ldv,
+                         (int)vt_stiles, (int)vt_dtiles, (int)gtiles, vt8);
+    else
+      hipLaunchKernelGGL(quant_group_kernel<kInBf16>, grid, block, 0, st, jobs, vt, ldv,
+                         (int)vt_stiles, (int)vt_dtiles, (int)gtiles, vt8);
+    return check_launch("quant_group");
+  }
   hipLaunchKernelGGL(amax_multi_kernel, dim3((unsigned)amax_blocks, 3), dim3(kQThreads), 0, st,
                      jobs);
   if ((rc = check_launch("amax_multi"))) return rc;
-  const int64_t vt_stiles = ldv / 128, vt_dtiles = (D + 63) / 64;
-  const int64_t vt_blocks = vt_stiles * vt_dtiles * B * H;
   // (with Q's codes, Q's own apply blocks write its scale; without them,
   // job 0's first blocks do, from any number of partials)
   const int64_t fold_blocks =

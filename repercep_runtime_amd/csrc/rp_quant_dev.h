@@ -268,15 +268,12 @@ __device__ __forceinline__ void apply_t_load(const QParams& p, float qm, int64_t
   }
 }
 
-// Second half: transpose the codes through `tile` and store the tile's rows.
-__device__ __forceinline__ void apply_t_store(const QParams& p, const uint32_t (&w)[4][2],
-                                              uint8_t* codes, int64_t ld, int64_t s_blk,
-                                              int64_t d_blk, int64_t bh, uint8_t* tile) {
-  const int64_t s0 = s_blk * 128;
-  const int64_t d0 = d_blk * 64;
-  const int dcols = (int)min((int64_t)64, p.D - d0);
-  const int q = threadIdx.x >> 3;
-  const int c = threadIdx.x & 7;
+// Second half: the transposed codes into `tile` (apply_t_put), and after a
+// barrier the tile's rows out of it (apply_t_out); `t` is the thread of the
+// tile's 256.
+__device__ __forceinline__ void apply_t_put(const uint32_t (&w)[4][2], uint8_t* tile, int t) {
+  const int q = t >> 3;
+  const int c = t & 7;
   // 4x4 byte transposes: rows i (s) x columns e (d) -> dword per column.
   const int qs = 4 * (q ^ (8 * (c & 3)));   // byte offset of this quad's dword in its row
 #pragma unroll
@@ -295,12 +292,19 @@ __device__ __forceinline__ void apply_t_store(const QParams& p, const uint32_t (
     *reinterpret_cast<uint32_t*>(&tile[(d + 2) * 128 + qs]) = col2;
     *reinterpret_cast<uint32_t*>(&tile[(d + 3) * 128 + qs]) = col3;
   }
-  __syncthreads();
+}
+
+__device__ __forceinline__ void apply_t_out(const QParams& p, uint8_t* codes, int64_t ld,
+                                            int64_t s_blk, int64_t d_blk, int64_t bh,
+                                            const uint8_t* tile, int t) {
+  const int64_t s0 = s_blk * 128;
+  const int64_t d0 = d_blk * 64;
+  const int dcols = (int)min((int64_t)64, p.D - d0);
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    const int dr = (threadIdx.x >> 3) + 32 * k;
+    const int dr = (t >> 3) + 32 * k;
     if (dr >= dcols) break;
-    const int ch = threadIdx.x & 7;
+    const int ch = t & 7;
     // physical 16-byte chunk ch of row dr holds the codes of s chunk
     // ch ^ 2((dr >> 3) & 3)
     const int sch = ch ^ (2 * ((dr >> 3) & 3));
@@ -309,6 +313,14 @@ __device__ __forceinline__ void apply_t_store(const QParams& p, const uint32_t (
         u32x4{v.x, v.y, v.z, v.w},
         reinterpret_cast<u32x4*>(codes + (bh * p.D + d0 + dr) * ld + s0 + sch * 16));
   }
+}
+
+__device__ __forceinline__ void apply_t_store(const QParams& p, const uint32_t (&w)[4][2],
+                                              uint8_t* codes, int64_t ld, int64_t s_blk,
+                                              int64_t d_blk, int64_t bh, uint8_t* tile) {
+  apply_t_put(w, tile, threadIdx.x);
+  __syncthreads();
+  apply_t_out(p, codes, ld, s_blk, d_blk, bh, tile, threadIdx.x);
 }
 
 template <int DT, bool NT>
