@@ -516,6 +516,14 @@ void attn_fwd_kernel(AttnArgs a) {
   static_assert(!MIXED || (OUT != kOutSplit && !WINDOW && !MULTI), "mixed launches");
   constexpr int QROWS = 32;
   constexpr int BLOCK_M = QROWS * NW;
+  // Where the row max of a tile's 64 scores per lane is taken: between the
+  // P.V MFMAs of its phase, or after them.  After is faster but for the
+  // multi-block launch at head dim 128 (per call, alternating on one box,
+  // between / after: 40 x 75600 54.86 / 54.53 ms; 16 x 20000 at D = 64 1310 /
+  // 1253 us and at D = 256 2330 / 2309; 16 x 16384 at D = 32 827 / 804; 16
+  // causal heads x 16384 654 / 641; multi-block 40 x 3600 at D = 64 183.3 /
+  // 181.4, at D = 128 240 / 244).
+  constexpr bool MAX_IN_PHASE = MULTI && DK == 128;
   // multi-block launches stage the next query block's Q in LDS: two buffers
   // of BLOCK_M rows (the block being switched to, and the one after)
   constexpr int Q_BYTES = MULTI ? BLOCK_M * DK : 0;
@@ -921,17 +929,14 @@ void attn_fwd_kernel(AttnArgs a) {
       // group 0 issues tile i+1; past the last tile it re-reads the last one
       // into the stages tile i+1 would use, which are free (see above)
       const TileDst nxt = tile_dst(min(i + 1, T - 1) % n_kb, i + 1);
-      // Without a window mask the row max is taken between the PV MFMAs, over
-      // the raw scores: rows past Skv duplicate key Skv-1, and the keys a
-      // shifted last tile repeats were in the tile before, so the raw max is
-      // the max over the tile's visible keys.  It is not when a shifted tile
-      // opens a key split (its repeats belong to the previous split), nor
-      // under a window mask: such a tile takes its max after the phase, from
-      // the masked scores.  (Taking it between the MFMAs there too, and again
-      // from the masked scores where the mask cuts the tile, was 2% slower at
-      // 16 causal heads x 16384: 654 against 641 us per call.)
+      // MAX_IN_PHASE: the row max is taken between the PV MFMAs, over the raw
+      // scores: rows past Skv duplicate key Skv-1, and the keys a shifted last
+      // tile repeats were in the tile before, so the raw max is the max over
+      // the tile's visible keys (but for a shifted tile that opens the range,
+      // which takes its max after the phase).  Else every tile takes its max
+      // after the phase, from the masked scores.
       float mh[8];
-      mfma_phase<DK, DV, LOADS, !WINDOW>(kl, vl, qop, pop, s, acc, alpha, mh, tl, nxt);
+      mfma_phase<DK, DV, LOADS, MAX_IN_PHASE>(kl, vl, qop, pop, s, acc, alpha, mh, tl, nxt);
       // the next block's Q, after the tile loads (so a counted wait can leave
       // it in flight)
       const bool q_issued = MULTI && LOADS && j == 0 && blk + 1 < nblk;
@@ -973,7 +978,7 @@ void attn_fwd_kernel(AttnArgs a) {
             }
         }
         float mx;
-        if (!WINDOW && !(j == 0 && tile_begin(0) != kv0)) {
+        if (MAX_IN_PHASE && !(j == 0 && tile_begin(0) != kv0)) {
           constexpr int NP = 2 * G::ETILES;   // partial maxima mh[0 .. NP)
           if constexpr (NP == 2) {
             mx = max3f(mh[0], mh[1], mh[1]);
