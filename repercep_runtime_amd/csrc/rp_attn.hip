@@ -503,8 +503,10 @@ __device__ __forceinline__ void mfma_phase(uint32_t kl, uint32_t vl,
 // before barrier 2j.  Only group 0 loads: the slot in which a group issues
 // loads costs its SIMD VALU time, and in this slot the MFMA group, not the
 // softmax group, has VALU time to spare.
+// WINDOW: a mask that cuts inside the key range (PREFIX: the shared-prefix
+// one, else the causal one).
 template <int DK, int DV, int OUT, bool WINDOW, bool MULTI, bool STAGE = false,
-          bool MIXED = false>
+          bool MIXED = false, bool PREFIX = false>
 __global__ __launch_bounds__(512, 1)
 void attn_fwd_kernel(AttnArgs a) {
   constexpr int NW = 8;
@@ -514,6 +516,7 @@ void attn_fwd_kernel(AttnArgs a) {
   static_assert(!STAGE || (MULTI && DK == 128 && (OUT == kOutBf16 || OUT == kOutF16)),
                 "staged output stores");
   static_assert(!MIXED || (OUT != kOutSplit && !WINDOW && !MULTI), "mixed launches");
+  static_assert(!PREFIX || WINDOW, "shared-prefix mask");
   constexpr int QROWS = 32;
   constexpr int BLOCK_M = QROWS * NW;
   // Where the row max of a tile's 64 scores per lane is taken: between the
@@ -593,7 +596,7 @@ void attn_fwd_kernel(AttnArgs a) {
   int bh = L / per_bh;
   int qb = MULTI ? (L - bh * per_bh) * a.qb_per_wg
                  : (L - bh * per_bh) / nsplit + first_qb;
-  if constexpr (WINDOW && OUT != kOutSplit) {
+  if constexpr (WINDOW && !PREFIX && OUT != kOutSplit) {
     if (a.longest_first) {
       // Causal blocks run longest first: block qb has about 2 qb + 2 key
       // tiles, and a launch in ascending order ends with its longest blocks
@@ -661,7 +664,7 @@ void attn_fwd_kernel(AttnArgs a) {
   const int kv_begin = split * a.split_tiles * kBlockN;
   const int kv_end = MIXED && !part ? a.Skv : min(a.Skv, kv_begin + a.split_tiles * kBlockN);
   int n_kb = (kv_end - kv_begin + kBlockN - 1) / kBlockN;
-  if (a.mask == RP_MASK_CAUSAL) {
+  if (WINDOW && !PREFIX) {
     const int q_last = min(q_block0 + BLOCK_M, a.Sq) - 1;
     n_kb = q_last < kv_begin ? 0 : min(n_kb, (q_last - kv_begin) / kBlockN + 1);
   }
@@ -945,19 +948,19 @@ void attn_fwd_kernel(AttnArgs a) {
       }
       if (i < T) {
         bool masked = tail;
-        if (a.mask == RP_MASK_CAUSAL) masked |= kv0 + kBlockN - 1 > q_wave0;
-        if (a.mask == RP_MASK_SHARED_PREFIX) masked |= kv0 + kBlockN > a.prefix;
+        if (WINDOW && !PREFIX) masked |= kv0 + kBlockN - 1 > q_wave0;
+        if (PREFIX) masked |= kv0 + kBlockN > a.prefix;
         if (masked) {
           // every supported mask is "kv < pre_end, or lo <= kv <= hi" with a
           // per-query window; bitwise predicates, one select per score
           const float ninf = -__builtin_inff();
           int lo = 0, hi = a.Skv - 1;
-          if (a.mask == RP_MASK_CAUSAL) hi = min(q, hi);
-          if (a.mask == RP_MASK_SHARED_PREFIX) {
+          if (WINDOW && !PREFIX) hi = min(q, hi);
+          if (PREFIX) {
             lo = a.prefix + q - q % a.suffix;
             hi = min(a.prefix + q, hi);
           }
-          const int pre_end = a.mask == RP_MASK_SHARED_PREFIX ? min(a.prefix, a.Skv) : 0;
+          const int pre_end = PREFIX ? min(a.prefix, a.Skv) : 0;
           // keys before kv0 are the shifted last tile's repeats
           const int kvl = tile_begin(j) + 32 * lg;
           const int lo_t = lo - kvl, hi_t = hi - kvl, pe_t = pre_end - kvl, new_t = kv0 - kvl;
@@ -966,13 +969,16 @@ void attn_fwd_kernel(AttnArgs a) {
   #pragma unroll
             for (int r = 0; r < 16; ++r) {
               const int o = 64 * (hh >> 1) + 16 * (hh & 1) + r;  // key - kvl
-              // Without a window lo is 0 and there is no prefix: two compares
-              // a score instead of four, and half the code of a path that
-              // runs once per block, its instructions uncached then (40 heads
-              // x 3600: the call 238.5 -> 230.5 us, 40 x 75600 54.35 -> 53.45
-              // ms).  (One compare, with a path of its own for key ranges
-              // shorter than a tile, made every copy of the loop spill.)
-              const int vis = WINDOW ? (o >= new_t) & (((o >= lo_t) & (o <= hi_t)) | (o < pe_t))
+              // But for the shared-prefix mask lo is 0 and there is no prefix:
+              // two compares a score instead of four, and half the code of a
+              // path that runs once or twice per block, its instructions
+              // uncached then (tail tiles, 40 heads x 3600: the call 238.5 ->
+              // 230.5 us, 40 x 75600 54.35 -> 53.45 ms; causal, 32 x 4096:
+              // 135.6 -> 130.6, 32 x 2048 66.4 ->
+              // 63.4).  (One compare for the tail, with a path of its
+              // own for key ranges shorter than a tile, made every copy of
+              // the loop spill.)
+              const int vis = PREFIX ? (o >= new_t) & (((o >= lo_t) & (o <= hi_t)) | (o < pe_t))
                                      : (o >= new_t) & (o <= hi_t);
               s[hh][r] = vis ? s[hh][r] : ninf;
             }
@@ -1152,7 +1158,10 @@ void launch_fwd(const AttnArgs& a, hipStream_t st) {
       return;
     }
   }
-  if (a.mask != RP_MASK_NONE)
+  if (a.mask == RP_MASK_SHARED_PREFIX)
+    hipLaunchKernelGGL((attn_fwd_kernel<D, DV, OUT, true, false, false, false, true>), grid, block,
+                       0, st, a);
+  else if (a.mask != RP_MASK_NONE)
     hipLaunchKernelGGL((attn_fwd_kernel<D, DV, OUT, true, false>), grid, block, 0, st, a);
   else
     hipLaunchKernelGGL((attn_fwd_kernel<D, DV, OUT, false, false>), grid, block, 0, st, a);
