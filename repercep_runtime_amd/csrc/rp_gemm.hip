@@ -67,6 +67,7 @@ struct GemmArgs {
   // slices of 128 per part, (M, N) per part
   float* part;
   int part_slices;
+  int band;   // gemm_mid_kernel: tiles of C walked down before the next column
 };
 
 // The batch a workgroup works on: offsets every operand pointer (one batch
@@ -891,6 +892,13 @@ int launch_mid(GemmArgs g, int64_t batch, int parts, hipStream_t st) {
     rp_set_error("gemm: grid too large");
     return RP_ERR_UNSUPPORTED;
   }
+  // Bands of eight tiles share B^T rows in an XCD's L2.  Row-scaled batches
+  // whose output is past twice the 256 MB cache -- the unfused attention's
+  // scores -- are bound by its way to HBM, and walk C row by row, so that
+  // whole rows leave together: 40 x 3600 x 3600 of K = 128 in the op 910 ->
+  // 875 us, 32 x 4096 x 4096 of K = 64 767 -> 753; smaller outputs lose
+  // (40 x 1024 x 3072 of K = 128 254 -> 260).
+  g.band = EPI == kEpiRows && 2.0 * (double)batch * (double)g.M * (double)g.N > 512e6 ? 1 : 8;
   hipLaunchKernelGGL((gemm_mid_kernel<BM, KN, EPI>),
                      dim3((unsigned)nwork, (unsigned)batch, (unsigned)parts), dim3(kG2Threads), 0,
                      st, g);

@@ -78,18 +78,17 @@ void gemm_mid_kernel(GemmArgs g) {
   const uint32_t smem_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
 
   gemm_batch(g);
-  // XCD-aware remap, then a column-major walk over 8-tile-tall bands of C
+  // XCD-aware remap, then a column-major walk over bands of C of g.band tiles
   const int nwork = g.tiles_m * g.tiles_n;
   const int w = blockIdx.x;
   const int per = nwork >> 3, rem = nwork & 7;
   const int xcd = w & 7;
   const int L = xcd * per + min(xcd, rem) + (w >> 3);
-  constexpr int kBand = 8;
-  const int band_tiles = kBand * g.tiles_n;
+  const int band_tiles = g.band * g.tiles_n;
   const int band = L / band_tiles;
   const int in_band = L - band * band_tiles;
-  const int band_h = min(kBand, g.tiles_m - band * kBand);
-  const int tm = band * kBand + in_band % band_h;
+  const int band_h = min(g.band, g.tiles_m - band * g.band);
+  const int tm = band * g.band + in_band % band_h;
   const int tn = in_band / band_h;
   const int64_t m0 = (int64_t)tm * BM;
   const int64_t n0 = (int64_t)tn * BN;
