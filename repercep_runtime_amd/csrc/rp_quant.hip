@@ -329,12 +329,20 @@ int check_launch(const char* what) {
   return RP_OK;
 }
 
-int launch_scale(const Plan& pl, float* dequant_out, void* ws, size_t ws_bytes, hipStream_t st) {
-  if (ws == nullptr || ws_bytes < pl.ws_bytes) {
-    rp_set_error("scale: workspace of %zu bytes needed, got %zu", pl.ws_bytes, ws_bytes);
-    return RP_ERR_WORKSPACE;
-  }
-  uint32_t* partial = static_cast<uint32_t*>(ws);
+QJob make_job(const Plan& pl, void* partial, float* dequant, uint8_t* codes) {
+  QJob jb{};
+  jb.p = pl.p;
+  jb.flat = pl.flat;
+  jb.per_bh = pl.per_bh;
+  jb.gsize = pl.gsize;
+  jb.nblocks = pl.p.ngroups * pl.p.nbg;
+  jb.partial = static_cast<uint32_t*>(partial);
+  jb.dequant = dequant;
+  jb.codes = codes;
+  return jb;
+}
+
+int launch_amax(const Plan& pl, uint32_t* partial, hipStream_t st) {
   const int64_t nblocks = pl.p.ngroups * pl.p.nbg;
   if (pl.flat)
     hipLaunchKernelGGL(amax_flat_kernel, dim3((unsigned)nblocks), dim3(kQThreads), 0, st, pl.p.x,
@@ -342,7 +350,35 @@ int launch_scale(const Plan& pl, float* dequant_out, void* ws, size_t ws_bytes, 
   else
     hipLaunchKernelGGL(amax_partial_kernel, dim3((unsigned)nblocks), dim3(kQThreads), 0, st,
                        pl.p, partial);
-  int rc = check_launch("amax_partial");
+  return check_launch("amax_partial");
+}
+
+// Scale and BHSD codes of one tensor with few partials per group: the apply
+// blocks fold them (job 0 of the multi-tensor launch), which saves the
+// finalize launch: FP8Linear over 512 x 5120 -> 5120 37.9 -> 36.9 us per call.
+int launch_scale_apply_fold(const Plan& pl, float* dequant_out, uint8_t* codes, void* ws,
+                            hipStream_t st) {
+  int rc = launch_amax(pl, static_cast<uint32_t*>(ws), st);
+  if (rc) return rc;
+  QJobs3 jobs{};
+  jobs.j0 = make_job(pl, ws, dequant_out, codes);
+  const dim3 grid((unsigned)jobs.j0.nblocks);
+  if (pl.dt == RP_DTYPE_F16)
+    hipLaunchKernelGGL(apply_fold_multi_kernel<kInF16>, grid, dim3(kQThreads), 0, st, jobs,
+                       QParams{}, 0, 0, 0, nullptr);
+  else
+    hipLaunchKernelGGL(apply_fold_multi_kernel<kInBf16>, grid, dim3(kQThreads), 0, st, jobs,
+                       QParams{}, 0, 0, 0, nullptr);
+  return check_launch("apply_fold");
+}
+
+int launch_scale(const Plan& pl, float* dequant_out, void* ws, size_t ws_bytes, hipStream_t st) {
+  if (ws == nullptr || ws_bytes < pl.ws_bytes) {
+    rp_set_error("scale: workspace of %zu bytes needed, got %zu", pl.ws_bytes, ws_bytes);
+    return RP_ERR_WORKSPACE;
+  }
+  uint32_t* partial = static_cast<uint32_t*>(ws);
+  int rc = launch_amax(pl, partial, st);
   if (rc) return rc;
   if (pl.dt == RP_DTYPE_F16)
     hipLaunchKernelGGL(scale_finalize_kernel<kInF16>, dim3((unsigned)pl.p.ngroups),
@@ -465,6 +501,9 @@ extern "C" int rp_fp8_scale_quantize(const void* x, int x_dtype, int64_t B, int6
     return RP_ERR_UNSUPPORTED;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (layout == RP_LAYOUT_BHSD && pl.p.nbg <= kFoldMaxPartials && workspace != nullptr &&
+      workspace_bytes >= pl.ws_bytes)
+    return launch_scale_apply_fold(pl, dequant_out, codes, workspace, st);
   rc = launch_scale(pl, dequant_out, workspace, workspace_bytes, st);
   if (rc) return rc;
   return launch_apply(pl, x, B, H, S, D, sb, sh, ss, dequant_out, codes, layout, ld, st);
@@ -522,16 +561,7 @@ static int qkv_launch(const Plan& pq, const Plan& pk, const Plan& pv, const void
   int rc;
   const int64_t ng = pq.p.ngroups;
   auto job = [&](const Plan& pl, size_t off, float* dq, uint8_t* codes) {
-    QJob jb{};
-    jb.p = pl.p;
-    jb.flat = pl.flat;
-    jb.per_bh = pl.per_bh;
-    jb.gsize = pl.gsize;
-    jb.nblocks = pl.p.ngroups * pl.p.nbg;
-    jb.partial = reinterpret_cast<uint32_t*>(ws + off);
-    jb.dequant = dq;
-    jb.codes = codes;
-    return jb;
+    return make_job(pl, ws + off, dq, codes);
   };
   QJobs3 jobs;
   jobs.j0 = job(pq, 0, dequant_out, q8);

@@ -55,3 +55,21 @@ def test_equals_single_tensor_calls(gpu: torch.device, case: tuple) -> None:
         assert torch.equal(a[~nan], b[~nan]) and bool(((a[nan] & 0x7F) == 0x7F).all())
         if lay == "bhds":
             assert bool((a[..., Skv:] == 0).all())
+
+
+@pytest.mark.parametrize("rows", [1, 511, 512, 513])
+@pytest.mark.parametrize("gran", ["tensor", "bh"])
+def test_single_tensor_scale_and_codes_around_the_fold(gpu: torch.device, rows: int,
+                                                       gran: str) -> None:
+    """One tensor with up to 256 partial maxima per group folds them in the
+    apply launch (512 rows of 8192), one more runs the finalize launch: both
+    equal the scale and the codes of separate calls."""
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    for permuted in (False, True):
+        x = torch.randn((1, rows, 2, 8192) if permuted else (1, 2, rows, 8192), generator=g,
+                        device=gpu).to(torch.bfloat16)
+        x = x.reshape(1, rows, 2 * 8, 1024).permute(0, 2, 1, 3) if permuted else x
+        dq, codes = ops.scale_quantize(x, gran)
+        ref = ops.per_bh_scale(x, gran)
+        assert torch.equal(dq, ref)
+        assert torch.equal(codes.view(torch.uint8), ops.quantize(x, ref, gran).view(torch.uint8))
