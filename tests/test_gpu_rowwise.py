@@ -236,3 +236,17 @@ def test_softmax_rowwise_quantize_widths(gpu: torch.device, cols: int, causal: b
     # long rows hold few distinct tiny codes near rounding boundaries: the
     # share of flips stays that of P values at a boundary, as above
     assert (gc == rc)[~nan].mean() > 0.999
+
+
+@pytest.mark.parametrize("shape", [(2, 8, 8), (3, 136, 72), (1, 64, 128), (2, 200, 264),
+                                   (1, 3600, 128), (2, 130, 72), (1, 72, 130)])
+def test_transpose16_widths_exact(gpu: torch.device, shape: tuple) -> None:
+    """The 16-byte transpose (R, C multiples of 8, ragged 64 x 64 tiles) and
+    the element one beside it, on the aligned tensor and one element into it."""
+    x = torch.randn(*shape).to(torch.bfloat16)
+    t = ops.transpose16(x.to(gpu))
+    assert torch.equal(t.cpu(), x.transpose(-1, -2).contiguous())
+    flat = torch.zeros(x.numel() + 1, dtype=torch.bfloat16, device=gpu)
+    view = flat[1:].view(shape)            # 2 bytes off alignment
+    view.copy_(x)
+    assert torch.equal(ops.transpose16(view).cpu(), x.transpose(-1, -2).contiguous())
