@@ -436,7 +436,8 @@ int rp_fp8_linear(const uint8_t* a8, const uint8_t* b8, int b_layout, const void
  * static shares ended 0.25 ms apart).  Every XCD runs its share of tiles
  * but the last few in place; the tiles so left are handed out, in share
  * order, through a counter in `workspace` to whichever XCD asks first.  The
- * outputs equal rp_fp8_linear's bit for bit.  workspace: at least
+ * outputs equal rp_fp8_linear's bit for bit (but for products split along K,
+ * which need more workspace: rp_fp8_linear_workspace_bytes).  workspace: at least
  * RP_GEMM_BALANCED_WORKSPACE_BYTES, 256-byte aligned, zeroed by the call's
  * own first kernel, not shared by calls that may overlap.  No counterpart
  * in the reference (its GEMM launch takes no workspace); for callers that

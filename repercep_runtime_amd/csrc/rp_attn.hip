@@ -403,7 +403,8 @@ __device__ __forceinline__ i32x8 lds_op(uint32_t lds_addr) {
 //   during S^T:  the loads of tile i+1 (LOADS) and O^T *= alpha(i-1), the
 //                rescale owed since the previous phase's row max (skipped
 //                when no row of the wave raised its max);
-//   during PV:   partial row maxima of S^T(i) (MAX), 64 / NP scores per step.
+//   during PV:   partial row maxima of S^T(i) (MAX), 64 / NP scores per step;
+//                most kernels take them after the phase (MAX_IN_PHASE).
 constexpr int kRing = 3;
 
 template <int DK, int DV, bool LOADS, bool MAX>

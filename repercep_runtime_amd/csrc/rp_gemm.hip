@@ -12,20 +12,24 @@
 // reference takes it, (K, N) row-major (RP_B_KN).  A (K, N) slice is staged
 // in LDS as it lies in memory -- K rows of N bytes -- and the B^T operand is
 // read from it with ds_read_b64_tr_b8, the gfx950 LDS transpose read (see
-// kn_operand), so neither layout costs a transpose pass.  Two kernels:
+// kn_operand), so neither layout costs a transpose pass.  Three kernels:
 //
-// * gemm256_kernel (K a multiple of 64, the production shapes): 256 x 256
+// * gemm256_kernel (K a multiple of 64, grids that fill the GPU): 256 x 256
 //   block tiles on v_mfma_f32_32x32x64_f8f6f4, four waves of 128 x 128 with
 //   their accumulators in AGPRs, operands streamed by direct-to-LDS loads
 //   through a ring of five 32 KiB slots (the A and B^T halves of 128-byte K
 //   slices), each slice loaded two slices ahead of its use.
+// * gemm_mid_kernel (rp_gemm_mid.h; any K multiple of 16): 128 x 128 or
+//   64 x 128 tiles through the same ring, K split over workgroups where M and
+//   N give few tiles.  gemm_plan chooses between the two.
 // * gemm_kernel (any K multiple of 16, any (K, N) B): 256 x 128 block tiles
 //   on v_mfma_f32_16x16x128_f8f6f4, operands staged through VGPRs into a
 //   double-buffered, XOR-swizzled LDS tile, K tail zero-filled; a (K, N) B
-//   is gathered byte by byte (the fallback for shapes the large-tile kernel
-//   does not take).
+//   is gathered byte by byte (the fallback for what the direct-to-LDS kernels
+//   do not take: an N or a base of a (K, N) B off 16 bytes, strides past
+//   their 32-bit tile offsets).
 //
-// Both remap workgroups so that those resident on one XCD cover a compact
+// All remap workgroups so that those resident on one XCD cover a compact
 // patch of C and share operand rows in that XCD's L2.
 
 #include <math.h>
