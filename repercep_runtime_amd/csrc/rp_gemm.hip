@@ -903,9 +903,12 @@ int launch_mid(GemmArgs g, int64_t batch, int parts, hipStream_t st) {
   // 875 us, 32 x 4096 x 4096 of K = 64 767 -> 753; smaller outputs lose
   // (40 x 1024 x 3072 of K = 128 254 -> 260).
   g.band = EPI == kEpiRows && 2.0 * (double)batch * (double)g.M * (double)g.N > 512e6 ? 1 : 8;
-  hipLaunchKernelGGL((gemm_mid_kernel<BM, KN, EPI>),
-                     dim3((unsigned)nwork, (unsigned)batch, (unsigned)parts), dim3(kG2Threads), 0,
-                     st, g);
+  const dim3 grid((unsigned)nwork, (unsigned)batch, (unsigned)parts);
+  const int64_t slices = EPI == kEpiPart ? g.part_slices : (g.K + kG2K - 1) / kG2K;
+  if (nwork * batch * parts <= kGmDeepGrid && slices >= kGmDeepSlices)
+    hipLaunchKernelGGL((gemm_mid_kernel<BM, KN, EPI, kGmDeep>), grid, dim3(kG2Threads), 0, st, g);
+  else
+    hipLaunchKernelGGL((gemm_mid_kernel<BM, KN, EPI, 2>), grid, dim3(kG2Threads), 0, st, g);
   if constexpr (EPI == kEpiPart) {
     const int64_t threads = g.M * (g.N / 4);
     hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,

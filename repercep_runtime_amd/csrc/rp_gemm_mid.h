@@ -7,9 +7,10 @@
 // v_mfma_f32_32x32x64_f8f6f4, four waves (2 x 2) of BM/2 x 64 each, C^T tiles
 // as in gemm256_kernel (A operand = rows of B^T).  Operands stream by
 // direct-to-LDS loads in K slices of 128 bytes through gemm256_kernel's ring
-// -- five slots, slice kk's A part in slot 2kk mod 5 and its B^T part in slot
-// 2kk + 1 mod 5, each slice loaded two slices ahead of its use -- but a slot
-// is 16 KiB, so two workgroups share a CU and one's waits, fill and stores
+// -- slice kk's A part in slot 2kk mod 5 and its B^T part in slot 2kk + 1
+// mod 5, each slice loaded two slices ahead of its use (mod 9 and four ahead
+// where a workgroup has its CU to itself, see LEAD) -- but a slot is 16 KiB,
+// so two workgroups share a CU and one's waits, fill and stores
 // overlap the other's MFMAs.
 //
 // What bounds it: a wave part of 64 x 64 reads (64 + 64) x 64 operand bytes
@@ -40,6 +41,22 @@ constexpr int kEpiPart = 3;   // fp32 partial sums of one K part (no scale)
 
 constexpr int kGmBN = 128;    // columns per tile
 
+// Slices loaded ahead of their use (LEAD): two in the five-slot ring, which
+// leaves LDS for a second workgroup on the CU.  A grid of at most a workgroup
+// per CU has that LDS to itself: nine slots, four slices ahead, for its loads
+// bound it (0.8 us per slice at two ahead when the operands come from HBM).
+// us per call, 2 / 4 ahead, weights changing from call to call, (N, K) and
+// (K, N) B: 256 x 5120 x 5120 32.3 / 23.8 and 40.1 / 30.1; 512 rows 33.9 /
+// 30.3 and 39.8 / 34.7; 256 x 4096 x 4096 25.9 / 17.6 and 26.6 / 21.4; 256 x
+// 3072 x 3072 13.9 / 11.0 and 14.6 / 12.6.  The same weights again and again:
+// 256 x 5120 x 5120 21.4 / 16.4, but 256 x 4096 x 4096, which the L2s hold,
+// 11.3 / 11.7.  Workgroups of few slices lose by the longer fill (16 x 4096 x
+// 4096, K parts of 4 slices, 9.1 / 9.7; 512 x 1536 x 8960, of 14, 20.0 /
+// 20.7).
+constexpr int kGmDeep = 4;
+constexpr int kGmDeepSlices = 20;
+constexpr int64_t kGmDeepGrid = 256;
+
 template <int BM>
 struct GmGeo {
   static constexpr int BN = kGmBN;
@@ -69,11 +86,19 @@ struct GmOps {
   i32x8 a[NBM], b[NBN];
 };
 
-template <int BM, bool KN, int EPI>
-__global__ __launch_bounds__(kG2Threads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// s_waitcnt vmcnt(max(n, 0)), n at most LOADS * MAX and a multiple of LOADS
+template <int LOADS, int MAX>
+__device__ __forceinline__ void gm_wait_slices(int left) {
+  if (MAX > 0 && left >= MAX) g2_wait_vmem<LOADS * MAX>();
+  else if constexpr (MAX > 0) gm_wait_slices<LOADS, MAX - 1>(left);
+  else g2_wait_vmem<0>();
+}
+
+template <int BM, bool KN, int EPI, int LEAD>
+__global__ __launch_bounds__(kG2Threads) __attribute__((amdgpu_waves_per_eu(LEAD > 2 ? 1 : 2, 2)))
 void gemm_mid_kernel(GemmArgs g) {
   using G = GmGeo<BM>;
-  constexpr int BN = kGmBN, SLOTS = kG2Slots, NBM = G::NBM, NBN = G::NBN, SLOT = G::SLOT;
+  constexpr int BN = kGmBN, SLOTS = 2 * LEAD + 1, NBM = G::NBM, NBN = G::NBN, SLOT = G::SLOT;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[SLOTS * SLOT];
   const uint32_t smem_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
 
@@ -189,14 +214,13 @@ void gemm_mid_kernel(GemmArgs g) {
     for (int j = 0; j < NBN; ++j) acc[i][j] = f32x16{};
 
 #pragma unroll
-  for (int n = 0; n < G::LOADS; ++n) issue(n, 0, n < G::ALOADS ? 0 : 1, std::false_type{});
-  if (nslice > 1) {
+  for (int s = 0; s < LEAD; ++s)
+    if (s < nslice) {
 #pragma unroll
-    for (int n = 0; n < G::LOADS; ++n) issue(n, 1, n < G::ALOADS ? 2 : 3, std::false_type{});
-    g2_wait_vmem<G::LOADS>();
-  } else {
-    g2_wait_vmem<0>();
-  }
+      for (int n = 0; n < G::LOADS; ++n)
+        issue(n, s, 2 * s + (n < G::ALOADS ? 0 : 1), std::false_type{});
+    }
+  gm_wait_slices<G::LOADS, LEAD - 1>(nslice - 1);   // slice 0 has landed
   __syncthreads();
   GmOps<NBM, NBN> o0, o1;
 #pragma unroll
@@ -217,7 +241,7 @@ void gemm_mid_kernel(GemmArgs g) {
 
   // Sub-step (kk, H), gemm256_kernel's schedule: the MFMAs of sub-slice
   // 2kk + H on `cur`, the operand reads of the next sub-slice into `nxt`
-  // (in the first half of the MFMAs) and the loads of slice kk + 2's A part
+  // (in the first half of the MFMAs) and the loads of slice kk + LEAD's A part
   // (H = 0) or B^T part (H = 1).  (kk, 1) begins with the slice's one wait and
   // barrier: slice kk + 1 has landed, and every wave has read slice kk.
   int sa = 0;   // slot of slice kk's A part
@@ -227,18 +251,19 @@ void gemm_mid_kernel(GemmArgs g) {
     constexpr bool STEADY = decltype(Sc)::value;
     const int u = 2 * kk + H;
     const bool more = STEADY || u + 1 < nsub;
-    const bool load = STEADY || kk + 2 < nslice;
+    const bool load = STEADY || kk + LEAD < nslice;
     if (!STEADY && !more && ktail < kG2Sub) zero_tail(cur);
     if (H == 1) {
       if (more) {
-        if (load) g2_wait_vmem<G::ALOADS>();
-        else g2_wait_vmem<0>();
+        // slices kk + 2 and on may stay in flight
+        if (load) g2_wait_vmem<(LEAD - 2) * G::LOADS + G::ALOADS>();
+        else gm_wait_slices<G::LOADS, LEAD - 2>(nslice - 2 - kk);
       }
       __syncthreads();
     }
     const uint8_t* sta = smem + (H == 0 ? sa : wrap(sa + 2)) * SLOT;
     const uint8_t* stb = smem + (H == 0 ? wrap(sa + 1) : wrap(sa + 3)) * SLOT;
-    const int lslot = H == 0 ? wrap(sa + 4) : sa;
+    const int lslot = H == 0 ? wrap(sa + 2 * LEAD) : sa;
     const int r0 = H == 0 ? h10 : h00, r1 = H == 0 ? h11 : h01;
     constexpr int NM = NBM * NBN;                        // MFMAs of the sub-step
     constexpr int NL = H == 0 ? G::ALOADS : G::BLOADS;   // loads
@@ -258,7 +283,7 @@ void gemm_mid_kernel(GemmArgs g) {
       if (load) {
 #pragma unroll
         for (int x = t * NL / NM; x < (t + 1) * NL / NM; ++x)
-          issue((H == 0 ? 0 : G::ALOADS) + x, kk + 2, lslot,
+          issue((H == 0 ? 0 : G::ALOADS) + x, kk + LEAD, lslot,
                 std::integral_constant<bool, STEADY>{});
       }
       if constexpr (STEADY) __builtin_amdgcn_sched_barrier(0);
@@ -269,7 +294,7 @@ void gemm_mid_kernel(GemmArgs g) {
   using H1 = std::integral_constant<int, 1>;
   const int nfull = nsub >> 1;
   int kk = 0;
-  const int nsteady = max(0, nslice - 3);
+  const int nsteady = max(0, nslice - 1 - LEAD);
   for (; kk < nsteady; ++kk) {
     sub(kk, H0{}, std::true_type{}, o0, o1);
     sub(kk, H1{}, std::true_type{}, o1, o0);

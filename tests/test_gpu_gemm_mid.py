@@ -34,6 +34,8 @@ def _codes(rows: int, cols: int, pad: int, gen: torch.Generator) -> torch.Tensor
     (64, 128, 64), (130, 128, 128), (127, 256, 192), (128, 128, 256),   # whole sub-slices
     (300, 400, 3600),                                              # the P.V product's K
     (16, 512, 4096), (100, 640, 8192), (17, 128, 2064),            # split K
+    (70, 144, 2448), (70, 144, 2608), (65, 128, 2624), (128, 256, 2816),   # 20 slices and on
+    (2050, 2064, 208), (2050, 2064, 752),                          # two tiles to a CU
 ])
 def test_edges_vs_exact(gpu: torch.device, M: int, N: int, K: int, bias: bool) -> None:
     g = torch.Generator().manual_seed(M + N + K)
@@ -97,7 +99,7 @@ def test_output_stride_and_untouched_padding(gpu: torch.device) -> None:
 
 
 @pytest.mark.parametrize("Z,M,N,K", [(2, 200, 128, 400), (3, 129, 64, 3600), (2, 300, 304, 128),
-                                     (1, 65, 96, 16)])
+                                     (1, 65, 96, 16), (50, 200, 300, 16), (50, 200, 300, 400)])
 def test_row_scaled_batches(gpu: torch.device, Z: int, M: int, N: int, K: int) -> None:
     """Row scales and batch strides: powers of two and small integers, exact."""
     g = torch.Generator().manual_seed(Z + M + N + K)
