@@ -483,10 +483,14 @@ int rp_fp8_transpose(const uint8_t* src, uint8_t* dst, int64_t R, int64_t C,
  * the CPU oracle.  They run the same device functions the kernels above use.
  * rp_selftest_e4m3: out[i] = e4m3fn code of clamp(x[i], -448, 448).
  * rp_selftest_scale: dequant[i] / qmul[i] from bf16 or fp16 (x_dtype) amax
- * bit patterns. */
+ * bit patterns.
+ * rp_selftest_rope_block (host only): the row range and the chunk of heads of
+ * block `block` of the prologue's rotary passes, of ranges * chunks blocks. */
 int rp_selftest_e4m3(const float* x, uint8_t* out, int64_t n, void* stream);
 int rp_selftest_scale(const uint16_t* amax_bits, int x_dtype, float* dequant, float* qmul, int64_t n,
                       void* stream);
+int rp_selftest_rope_block(int64_t ranges, int64_t chunks, int64_t block, int64_t* range,
+                           int64_t* chunk);
 
 #ifdef __cplusplus
 }

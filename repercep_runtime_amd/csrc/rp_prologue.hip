@@ -395,9 +395,9 @@ __device__ __forceinline__ void prologue_quant_body(const PParams& p, int64_t bl
 // block, as the plain rows run, every head reads the whole fp32 (S, D)
 // tables again -- 64 bytes of L2 / MALL traffic per 16 bytes of input, 3.7 GB
 // per pass over Q and K at (1, 32, 56320, 128), which was the pass's time;
-// eight heads per block leave 8 bytes per 16.  Row ranges that lie eight
-// apart in block order share an XCD's L2, so the chunks of one range find
-// its tables there.
+// eight heads per block leave 8 bytes per 16.  The chunks of one range run on
+// one XCD as far as that fills all eight (rope_block), and find its tables in
+// that XCD's L2.
 //
 // D/16 threads share a row; thread c holds 16-byte chunks c and c + D/16,
 // that is elements d and their half-rotation partners d + D/2: neither
@@ -413,8 +413,13 @@ __device__ __forceinline__ void prologue_quant_body(const PParams& p, int64_t bl
 // chunk per thread, 0.674 ms here; 4 or 16 heads per block 0.692 / 0.675 ms.
 constexpr int kRopeMaxHeads = 16;   // LDS words for a block's heads
 constexpr int kRopeHeads = 8;       // heads per block
-// Fewer heads per block below this many blocks (per tensor): at
+// Fewer heads per block, down to two, below this many blocks (per tensor): at
 // (1, 40, 16384, 128) 1024 and 256 take 0.264 and 0.267 ms, 3000 0.284 ms.
+// Calls of 64 to 2048 positions reach the floor of two heads and are no
+// slower with it than with a head per block and chunk per thread (Q, K and V,
+// us: (1, 40, 512, 128) 27.4 / 22.4, (2, 16, 256, 64) 20.8 / 19.8,
+// (8, 32, 1024, 128) 149 / 113); of up to 8 positions they are, by 1.0-1.9 us
+// of GPU time (8.4 / 9.7 at (1, 40, 1, 64)), which eager launches hide.
 constexpr int64_t kRopeMinBlocks = 1024;
 
 // two fp32 -> their nearest-even bf16 values as fp32 (one v_cvt_pk_bf16_f32)
@@ -482,6 +487,26 @@ __device__ __forceinline__ uint32_t rope_row(float (&x)[16], float r, bool has_w
   return m;
 }
 
+// The row range and head chunk of block b, b < ranges * chunks.  Blocks go to
+// the XCDs in turn (b % 8).  Of whole groups of eight ranges each XCD takes
+// one range, its chunks one after another; the chunks of what is left are
+// dealt out in eight equal runs, so that neighbours on an XCD share a range.
+// (With every range on one XCD, a call of fewer than eight ranges ran on as
+// many XCDs, and nine ranges took two turns on one of them.  Q, K and V in a
+// call, us: (8, 32, 64, 128) 33.1 -> 18.8; (8, 32, 512, 64) 66.1 -> 37.5;
+// (1, 40, 512, 128) 27.8 -> 22.4; whole groups of eight the same.  With a
+// head per block, before the tables were kept in registers: 20.8, 47.6, 27.4.)
+struct RopeBlock {
+  uint32_t range, chunk;
+};
+__host__ __device__ inline RopeBlock rope_block(uint32_t b, uint32_t ranges, uint32_t chunks) {
+  const uint32_t xcd = b & 7, q = b >> 3, whole = (ranges >> 3) * chunks;
+  if (q < whole) return {q / chunks * 8 + xcd, q % chunks};
+  const uint32_t left = (ranges & 7) * chunks, rem = left & 7;
+  const uint32_t L = xcd * (left >> 3) + (xcd < rem ? xcd : rem) + (q - whole);
+  return {(ranges & ~7u) + L / chunks, L % chunks};
+}
+
 // Block b of one tensor.  APPLY: codes under the given scales; else the
 // partial maxima, one per (head, row range).
 template <int D, int ROPE, bool APPLY>
@@ -494,11 +519,10 @@ __device__ __forceinline__ void rope_body(const PParams& p, int64_t b, uint32_t*
   constexpr int U = 2;                           // heads side by side
   __shared__ uint32_t s_max[kRopeMaxHeads];
   __shared__ float s_qm[kRopeMaxHeads];
-  const int64_t q = b >> 3;
-  const int64_t hcI = q % p.nhc;
-  const int64_t sr = (q / p.nhc) * 8 + (b & 7);
-  if (sr >= p.nsr) return;
-  const int bh0 = (int)hcI * p.hc;
+  const RopeBlock rb = rope_block((uint32_t)b, (uint32_t)p.nsr, (uint32_t)p.nhc);
+  const int64_t sr = rb.range;
+  const int hcI = (int)rb.chunk;
+  const int bh0 = hcI * p.hc;
   const int nh = min(p.hc, (int)(p.B * p.H) - bh0);
   if ((int)threadIdx.x < nh) {
     if constexpr (APPLY) s_qm[threadIdx.x] = 1.0f / dequant[per_bh ? bh0 + threadIdx.x : 0];
@@ -693,7 +717,7 @@ int launch_check(const char* what) {
 
 // Blocks of one tensor's pass.
 inline int64_t prologue_blocks(const PParams& p, int64_t ngroups) {
-  return p.cosv != nullptr ? (p.nsr + 7) / 8 * 8 * p.nhc : ngroups * p.nbg;
+  return p.cosv != nullptr ? p.nsr * p.nhc : ngroups * p.nbg;
 }
 
 template <int D, int ROPE>
@@ -835,6 +859,19 @@ int with_layout(int64_t D, int rope_mode, F&& f) {
 }  // namespace rp
 
 using namespace rp;
+
+extern "C" int rp_selftest_rope_block(int64_t ranges, int64_t chunks, int64_t block,
+                                      int64_t* range, int64_t* chunk) {
+  if (range == nullptr || chunk == nullptr || ranges <= 0 || chunks <= 0 ||
+      ranges > 0x7fffffff / chunks || block < 0 || block >= ranges * chunks) {
+    rp_set_error("selftest_rope_block: bad arguments");
+    return RP_ERR_INVALID_ARGUMENT;
+  }
+  const RopeBlock rb = rope_block((uint32_t)block, (uint32_t)ranges, (uint32_t)chunks);
+  *range = rb.range;
+  *chunk = rb.chunk;
+  return RP_OK;
+}
 
 extern "C" size_t rp_fp8_rmsnorm_quant_workspace_bytes(int64_t B, int64_t H, int64_t S, int64_t D,
                                                        int granularity) {

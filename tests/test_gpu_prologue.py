@@ -231,3 +231,23 @@ def test_rotary_head_chunks_equal_single_heads(gpu: torch.device, rope: str, gra
         top = max(range(H), key=lambda h: float(one[h][0]))
         assert float(dq) == float(one[top][0])
         assert torch.equal(codes[:, top].view(torch.uint8), one[top][1][:, 0].view(torch.uint8))
+
+
+@pytest.mark.parametrize("B,H,S,D,rope", [
+    (1, 5, 1, 128, "half"),             # one row: one range, three chunks
+    (2, 33, 300, 128, "interleaved"),   # three ranges, 33 chunks of two heads
+    (3, 3, 2200, 64, "half"),           # nine ranges: a group of eight and one more
+])
+def test_rotary_few_ranges_equal_single_heads(gpu: torch.device, B: int, H: int, S: int, D: int,
+                                              rope: str) -> None:
+    """Ranges that do not fill groups of eight: every head's scale and codes
+    equal those of a call on that head alone (one chunk)."""
+    x = _x(B + H + S, (B, H, S, D), 2.0).to(gpu)
+    w = _x(6, (D,), 0.8).to(gpu)
+    t = tuple(torch.from_numpy(a).to(gpu) for a in _tables(S, D))
+    dq, codes = ops.rmsnorm_scale_quantize(x, w, 1e-6, t, rope, "bh")
+    for b in range(B):
+        for h in range(H):
+            d, c = ops.rmsnorm_scale_quantize(x[b:b + 1, h:h + 1], w, 1e-6, t, rope, "bh")
+            assert torch.equal(dq.view(B, H)[b, h], d[0])
+            assert torch.equal(codes[b, h].view(torch.uint8), c[0, 0].view(torch.uint8))
