@@ -484,11 +484,15 @@ int rp_fp8_transpose(const uint8_t* src, uint8_t* dst, int64_t R, int64_t C,
  * rp_selftest_e4m3: out[i] = e4m3fn code of clamp(x[i], -448, 448).
  * rp_selftest_scale: dequant[i] / qmul[i] from bf16 or fp16 (x_dtype) amax
  * bit patterns.
+ * rp_selftest_quant_one_launch (host only): 1 where a Q/K/V quantizer call of
+ * `groups` groups of up to `elems` (<= 65536) elements and `tiles` (<= 8) V^T
+ * tiles of 128 x 64 takes one launch.
  * rp_selftest_rope_block (host only): the row range and the chunk of heads of
  * block `block` of the prologue's rotary passes, of ranges * chunks blocks. */
 int rp_selftest_e4m3(const float* x, uint8_t* out, int64_t n, void* stream);
 int rp_selftest_scale(const uint16_t* amax_bits, int x_dtype, float* dequant, float* qmul, int64_t n,
                       void* stream);
+int rp_selftest_quant_one_launch(int64_t groups, int64_t elems, int64_t tiles, int capturing);
 int rp_selftest_rope_block(int64_t ranges, int64_t chunks, int64_t block, int64_t* range,
                            int64_t* chunk);
 

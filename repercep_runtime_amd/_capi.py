@@ -54,7 +54,8 @@ EXPORTS = (
     "rp_fp8_linear_balanced", "rp_fp8_linear_workspace_bytes", "rp_fp8_transpose",
     "rp_fp8_gemm_rowwise", "rp_fp8_rowwise_quantize", "rp_transpose16",
     "rp_fp8_softmax_rowwise_quantize",
-    "rp_selftest_e4m3", "rp_selftest_scale", "rp_selftest_rope_block",
+    "rp_selftest_e4m3", "rp_selftest_scale", "rp_selftest_quant_one_launch",
+    "rp_selftest_rope_block",
 )
 
 
@@ -166,6 +167,8 @@ def _declare(L: ctypes.CDLL) -> None:
     L.rp_selftest_e4m3.argtypes = [_vp, _vp, _i64, _vp]
     L.rp_selftest_scale.restype = _int
     L.rp_selftest_scale.argtypes = [_vp, _int, _vp, _vp, _i64, _vp]
+    L.rp_selftest_quant_one_launch.restype = _int
+    L.rp_selftest_quant_one_launch.argtypes = [_i64, _i64, _i64, _int]
     L.rp_selftest_rope_block.restype = _int
     L.rp_selftest_rope_block.argtypes = [_i64, _i64, _i64, ctypes.POINTER(_i64), ctypes.POINTER(_i64)]
 

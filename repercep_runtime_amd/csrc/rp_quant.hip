@@ -82,7 +82,7 @@ struct QJob {
   QParams p;          // the tensor's plan
   int flat;           // contiguous: the flat kernels
   int per_bh;
-  int64_t gsize;      // elements per group (flat)
+  int64_t gsize;      // elements per group
   int64_t nblocks;    // ngroups * nbg
   uint32_t* partial;  // this job's partial maxima
   float* dequant;     // this job's scales
@@ -181,12 +181,7 @@ __global__ __launch_bounds__(kQThreads) void apply_fold_multi_kernel(QJobs3 jobs
 // per thread), reduces its maximum, computes its scale and quantizes what it
 // holds -- one launch, no partial maxima, no second read.  V^T's groups are
 // held as the 128 x 64 tiles of the transposing apply, four at a time.
-// The host's launches bound calls this small, so the launch saved is what
-// counts: attention over (1, 8, 1024, 64) takes 23.1 us per call against
-// 26.9 with the amax and folded apply launches, (2, 40, 512, 128) 30.8
-// against 38.0.  On the GPU one CU per group is just level with those two at
-// 65536 elements (10.3 us against 3.7 + 5.7 and a gap: ~6 VALU instructions
-// per element on one CU) and behind past it (131072: 17.1 against 3.6 + 5.5).
+// Which calls take it: one_launch_pays.
 constexpr int kGroupThreads = 1024;
 constexpr int kGroupVecs = 8;        // 16-byte vectors per thread: 65536 elements per group
 
@@ -351,6 +346,34 @@ int launch_amax(const Plan& pl, uint32_t* partial, hipStream_t st) {
     hipLaunchKernelGGL(amax_partial_kernel, dim3((unsigned)nblocks), dim3(kQThreads), 0, st,
                        pl.p, partial);
   return check_launch("amax_partial");
+}
+
+// Whether a Q/K/V call of `groups` groups of up to `elems` elements and
+// `tiles` V^T tiles each, which fit quant_group_kernel, runs in its one launch.  GPU time in us, two launches
+// (amax_multi, apply_fold_multi) / one (contiguous Q, K, V; groups x elements):
+//    8 x 1024    6.7 / 7.0       8 x 32768   7.8 / 7.4      640 x 1024   10.7 / 21.7
+//   40 x 8192    8.5 / 7.2      80 x 32768  11.9 / 8.4      640 x 8192   18.3 / 23.6
+//    8 x 65536   7.9 / 9.8     320 x 32768  29.0 / 20.5    2560 x 8192   58.6 / 74.2
+//   16 x 65536   9.7 / 10.1     40 x 65536  12.3 / 11.2    2560 x 16384   102 / 91
+// One CU per group is slower where it has a whole group of 65536 to convert
+// (or eight V^T tiles, full or not) and the others wait, and where so small a group leaves most of its 1024
+// threads idle that the groups queue.  An eager call is bound by its launches:
+// it takes 25-26 us in two and 22-23 in one (8 to 160 groups of any size), so
+// there the saved launch counts, up to as many workgroups as run at once (two
+// per CU); a captured graph replays without the host, so its GPU time counts.
+bool one_launch_pays(int64_t groups, int64_t elems, int64_t tiles, bool capturing) {
+  const bool threads_busy = elems >= 16384 || (elems >= 8192 && groups <= 170);
+  const bool cus_busy = max(elems, tiles * 128 * 64) <= 32768 || groups >= 32;
+  return (threads_busy && cus_busy) || (!capturing && 3 * groups <= 2 * 256);
+}
+
+bool is_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+    (void)hipGetLastError();   // the launch that follows reports its own error
+    return false;
+  }
+  return cap != hipStreamCaptureStatusNone;
 }
 
 // Scale and BHSD codes of one tensor with few partials per group: the apply
@@ -552,7 +575,8 @@ static int qkv_plan(const void* q, const void* k, const void* v, int x_dtype, in
   return RP_OK;
 }
 
-// The four launches of one Q/K/V quantizer call, partial maxima in `ws`.
+// The launches of one Q/K/V quantizer call (one, two or four), partial maxima
+// in `ws`.
 static int qkv_launch(const Plan& pq, const Plan& pk, const Plan& pv, const void* v,
                       int x_dtype, int64_t B, int64_t H, int64_t Skv, int64_t D, int64_t vsb,
                       int64_t vsh, int64_t vss, float* dequant_out, uint8_t* q8, uint8_t* k8,
@@ -576,9 +600,10 @@ static int qkv_launch(const Plan& pq, const Plan& pk, const Plan& pv, const void
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t vt_stiles = ldv / 128, vt_dtiles = (D + 63) / 64;
   const int64_t vt_blocks = vt_stiles * vt_dtiles * B * H;
-  // groups that fit one workgroup's registers: one launch
+  // groups that fit one workgroup's registers: one launch where that pays
   const int64_t gmax = max(pq.gsize, pk.gsize), gtiles = vt_blocks / ng;
-  if (q8 != nullptr && gmax <= (int64_t)kGroupThreads * 8 * kGroupVecs && gtiles <= kGroupVecs) {
+  if (q8 != nullptr && gmax <= (int64_t)kGroupThreads * 8 * kGroupVecs && gtiles <= kGroupVecs &&
+      one_launch_pays(ng, gmax, gtiles, is_capturing(st))) {
     QParams vt{};
     vt.x = static_cast<const uint16_t*>(v);
     vt.B = B; vt.H = H; vt.S = Skv; vt.D = D; vt.sb = vsb; vt.sh = vsh; vt.ss = vss;
@@ -756,6 +781,11 @@ extern "C" int rp_fp8_scale_quantize_qkv_noalloc(const void* q, const void* k, c
   if ((rc = scratch_for_stream(st, &ws))) return rc;
   return qkv_launch(pq, pk, pv, v, x_dtype, B, H, Skv, D, vsb, vsh, vss, dequant_out, q8, k8,
                     vt8, ldv, ws, off_k, off_v, stream);
+}
+
+extern "C" int rp_selftest_quant_one_launch(int64_t groups, int64_t elems, int64_t tiles,
+                                            int capturing) {
+  return one_launch_pays(groups, elems, tiles, capturing != 0) ? 1 : 0;
 }
 
 extern "C" int rp_selftest_e4m3(const float* x, uint8_t* out, int64_t n, void* stream) {

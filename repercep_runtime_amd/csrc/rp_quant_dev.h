@@ -340,7 +340,7 @@ struct Plan {
   int per_bh;
   size_t ws_bytes;
   bool flat;      // contiguous input: the flat kernels apply
-  int64_t gsize;  // elements per group when flat
+  int64_t gsize;  // elements per group
 };
 
 bool is_pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
