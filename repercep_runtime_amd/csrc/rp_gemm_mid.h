@@ -3,7 +3,7 @@
 // Included by rp_gemm.hip, whose helpers (GemmArgs, the direct-to-LDS load,
 // the MFMA and epilogue functions) it uses.
 //
-// gemm_mid_kernel<BM, KN, EPI>: block tiles of BM x 128 (BM 128 or 64) on
+// gemm_mid_kernel<BM, KN, EPI, LEAD>: block tiles of BM x 128 (BM 128 or 64) on
 // v_mfma_f32_32x32x64_f8f6f4, four waves (2 x 2) of BM/2 x 64 each, C^T tiles
 // as in gemm256_kernel (A operand = rows of B^T).  Operands stream by
 // direct-to-LDS loads in K slices of 128 bytes through gemm256_kernel's ring
@@ -403,9 +403,14 @@ void gemm_mid_kernel(GemmArgs g) {
     if (c16 && n + 8 <= g.N) {
       __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(dst));
     } else {
-      __builtin_nontemporal_store(u32x2{t.x, t.y}, reinterpret_cast<u32x2*>(dst));
+      // rows off 16 bytes share their cache lines with the neighbouring tile:
+      // kept in L2, the halves of a line leave together (non-temporal / plain,
+      // us: 40 x 2500 x 2500 of K = 64 420 / 235, 8 x 2500 x 2500 81 / 39,
+      // 20000 x 3076 of K = 512 102 / 60; 40 x 2500 x 2500 of K = 512 loses,
+      // 294 / 343, and takes the large tiles, 300)
+      *reinterpret_cast<u32x2*>(dst) = u32x2{t.x, t.y};
       if (n + 8 <= g.N)   // N % 4 == 0
-        __builtin_nontemporal_store(u32x2{t.z, t.w}, reinterpret_cast<u32x2*>(dst + 4));
+        *reinterpret_cast<u32x2*>(dst + 4) = u32x2{t.z, t.w};
     }
   }
 }
