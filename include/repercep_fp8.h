@@ -456,6 +456,15 @@ int rp_fp8_linear_balanced(const uint8_t* a8, const uint8_t* b8, int b_layout, c
  * and the two results differ by the order of their fp32 sums). */
 size_t rp_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
+/* How the products above run on operands that the direct-to-LDS kernels take
+ * (host only): *tile_rows 256 (256 x 256 tiles), 128 or 64 (x 128 columns),
+ * *k_parts the parts of a split K (may_split: rp_fp8_linear_balanced with the
+ * workspace above; else 1), *slices_ahead the 128-byte K slices loaded ahead.
+ * C is taken as packed and 16-byte aligned; batch 1 but for
+ * rp_fp8_gemm_rowwise. */
+int rp_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int may_split,
+                     int* tile_rows, int* k_parts, int* slices_ahead);
+
 /* rp_fp8_gemm with row-wise scales, batched: for each batch z < `batch`,
  *   C_z (M, N) = bf16( fp32(fp32(A8_z . B8_z) * row_scale_z[m]) * col_scale_z[n] )
  * with A8_z = a8 + z*bsa, B8_z = b8 + z*bsb (bytes), C_z = c + z*bsc,

@@ -51,7 +51,8 @@ EXPORTS = (
     "rp_fp8_rmsnorm_quant_workspace_bytes",
     "rp_fp8_rmsnorm_scale_quantize", "rp_fp8_rmsnorm_quant_qkv_workspace_bytes",
     "rp_fp8_rmsnorm_scale_quantize_qkv", "rp_fp8_gemm", "rp_fp8_linear",
-    "rp_fp8_linear_balanced", "rp_fp8_linear_workspace_bytes", "rp_fp8_transpose",
+    "rp_fp8_linear_balanced", "rp_fp8_linear_workspace_bytes", "rp_fp8_gemm_plan",
+    "rp_fp8_transpose",
     "rp_fp8_gemm_rowwise", "rp_fp8_rowwise_quantize", "rp_transpose16",
     "rp_fp8_softmax_rowwise_quantize",
     "rp_selftest_e4m3", "rp_selftest_scale", "rp_selftest_quant_one_launch",
@@ -151,6 +152,8 @@ def _declare(L: ctypes.CDLL) -> None:
     L.rp_fp8_linear_balanced.argtypes = (list(L.rp_fp8_linear.argtypes[:-1]) + [_vp, _sz, _vp])
     L.rp_fp8_linear_workspace_bytes.restype = _sz
     L.rp_fp8_linear_workspace_bytes.argtypes = [_i64, _i64, _i64]
+    L.rp_fp8_gemm_plan.restype = _int
+    L.rp_fp8_gemm_plan.argtypes = [_i64] * 4 + [_int] + [ctypes.POINTER(_int)] * 3
     L.rp_fp8_gemm_rowwise.restype = _int
     L.rp_fp8_gemm_rowwise.argtypes = ([_vp, _vp, _int, _vp] + [_i64] * 6 + [_vp, _vp]
                                       + [_i64] * 6 + [_vp])

@@ -832,33 +832,73 @@ struct GemmPlan {
   int part_slices = 0;   // 128-byte K slices per part
 };
 
-// The plan of a product that both kernels can run (whole = K % 64 == 0; only
-// the medium tiles take another K), from estimated times in us:
-// * 256 x 256 tiles run in rounds of one per CU: 1.45 per K slice and round
-//   and 4 for a tile's fill and stores (measured 60 for 40 slices);
+// Whether a product whose 128 x 128 tiles (t128 of them, t256 of 256 x 256)
+// do not run all at once, two to a CU, takes them all the same.  Measured over
+// 429 such products with N a multiple of 8 -- nine projections of M 512 ..
+// 24000 in both layouts, the same weights again and weights from HBM, and
+// batches of K 64 .. 4096 -- as the medium tiles' time over the large ones':
+// * K up to 512: 0.64-0.99; past it the medium tiles' operand reads show, and
+//   a large grid loses: 40 x 4096 x 4096 of K = 512 / 1024 / 2048 0.94 / 1.12 /
+//   1.31.
+// * Large tiles that run in one round (t256 <= 256): the gain ends between K
+//   of 1024 and 2048 (8192 x 1536 0.74 and 0.88, 1500 x 8960 of 1536 0.96-1.12),
+//   in a batch at 512 (40 x 512 x 512 of K = 512 / 1024 1.04 / 1.14); 2048 x 5120
+//   x 5120 1.03-1.34, 2048 x 5120 x 13824 1.06-1.54, the worst with weights from
+//   HBM.
+// * More rounds, the last nearly empty: 3600 x 5120 x 5120 (1.17 rounds) 0.88,
+//   1300 x 11008 x 4096 (1.01) 0.68-0.82, 8192 x 3072 x 3072 (1.50) 0.93, 6000
+//   x 5120 x 5120 (1.88) 1.19.  The two estimates (us) are fits; batches,
+//   weights past 40 MB and more than four rounds ask for a gain, for there
+//   the medium tiles' is too low.
+// * C rows off 16 bytes, past the 256 MB cache: the medium tiles' stores lose
+//   (40 x 2500 x 2500 of K = 256 / 512 1.06 / 1.14).
+// Of the 429 a handful take the slower form, by 5% at the most.
+inline bool medium_pays(int64_t M, int64_t N, int64_t K, int64_t batch, double t128, double t256,
+                        bool wide_c) {
+  const double ns = (double)((K + kG2K - 1) / kG2K);
+  if (!wide_c && 2.0 * (double)batch * (double)M * (double)N > 256e6) return false;
+  if (ns <= 4) return true;
+  if (t256 <= 256.0) return ns <= 8 && batch == 1;
+  const double rounds = ceil(t256 / 256.0), fill = t256 / (256.0 * rounds);
+  const double large = rounds * (ns * (0.70 + 0.60 * fill) + 13.5 - 2.0 * fill);
+  const double medium = 0.43 * ns * (t128 / 256.0 + 0.42) + 2.0 * t128 / 256.0 + 2.5;
+  const bool far = t256 > 1024.0 || (double)N * (double)K > 40e6;
+  return medium < (far ? 0.9 : batch > 1 ? 0.95 : 1.04) * large;
+}
+
+// The plan of a product that the direct-to-LDS kernels can run (whole = K %
+// 64 == 0: only the medium tiles take another K; wide_c: 16-byte C rows).
+// Medium tiles that all run at once beat the large ones (0.14-0.96 of their
+// time over the projections; batches with K of 3584 and 4096 0.9-1.07);
+// medium_pays decides the rest.
+// Among the medium forms, from estimated times in us:
 // * 128 x 128 tiles: 0.465 per slice and tile of each CU's share, the share
 //   taken as half a tile more than the mean (they run two to a CU), at least
 //   1.25 tiles' time (one alone does not fill the CU);
-// * 64 x 128 tiles 0.32, and better than 128 x 128 only where every tile has
-//   a CU to itself (256 x 5120 x 5120: 21.6 against 22.9 us; 512 rows, 320
-//   tiles: 25.1 against 23.2);
+// * 64 x 128 tiles 0.32, only where every tile has a CU to itself;
 // * a wave of few tiles waits for its loads, at least 0.45 per slice;
 // * K parts write and read fp32 sums (about 3.5 TB/s) and take another
 //   launch, ~5.5.
-// The constants are fits to a sweep over M 16 .. 16384 of seven projection
-// shapes (a few of its rows stand in rp_gemm_mid.h); where the two kernels'
-// estimates cross they lie within ~4% of each other.
+// These constants are fits to the two-ahead ring with (N, K) weights used
+// again and again, over M 16 .. 16384 of seven projections.  The four-ahead
+// ring, (K, N) weights and weights from HBM are not modelled: over the nine
+// projections the choice is within 4% of the best form in four products of
+// five, and at worst 1.36 times it (700 x 1536 x 8960 with weights from HBM,
+// 32.6 against 23.9 us).
 // A row-scaled (batched) product is never split; nor one whose caller brings
-// no workspace (may_split).
+// no workspace (may_split).  The CU count is the MI355X's.
 inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool whole,
-                          bool may_split) {
+                          bool may_split, bool wide_c) {
   constexpr double kCu = 256.0;
   const double ns = (double)((K + kG2K - 1) / kG2K);
   auto tiles = [&](int bm, int bn) {
     return (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn) * (double)batch;
   };
   GemmPlan best;
-  double cost = whole ? ceil(tiles(256, 256) / kCu) * (1.45 * ns + 4.0) : 1e30;
+  const double t128 = tiles(128, kGmBN);
+  if (whole && t128 > 2 * kCu && !medium_pays(M, N, K, batch, t128, tiles(256, 256), wide_c))
+    return best;
+  double cost = 1e30;
   for (int bm = 128; bm >= 64; bm -= 64) {
     const double t = tiles(bm, kGmBN);
     if (bm == 64 && t > kCu) break;
@@ -887,6 +927,12 @@ inline size_t gemm_workspace_bytes(int64_t M, int64_t N, const GemmPlan& p) {
          (p.parts > 1 ? (size_t)p.parts * (size_t)M * (size_t)N * sizeof(float) : 0);
 }
 
+// Slices a medium-tile launch loads ahead (see kGmDeep).
+inline int mid_lead(int64_t M, int64_t N, int64_t batch, int bm, int parts, int64_t slices) {
+  const int64_t nwork = ((M + bm - 1) / bm) * ((N + kGmBN - 1) / kGmBN);
+  return nwork * batch * parts <= kGmDeepGrid && slices >= kGmDeepSlices ? kGmDeep : 2;
+}
+
 template <int BM, bool KN, int EPI>
 int launch_mid(GemmArgs g, int64_t batch, int parts, hipStream_t st) {
   g.tiles_m = (int)((g.M + BM - 1) / BM);
@@ -899,13 +945,14 @@ int launch_mid(GemmArgs g, int64_t batch, int parts, hipStream_t st) {
   // Bands of eight tiles share B^T rows in an XCD's L2.  Row-scaled batches
   // whose output is past twice the 256 MB cache -- the unfused attention's
   // scores -- are bound by its way to HBM, and walk C row by row, so that
-  // whole rows leave together: 40 x 3600 x 3600 of K = 128 in the op 910 ->
-  // 875 us, 32 x 4096 x 4096 of K = 64 767 -> 753; smaller outputs lose
-  // (40 x 1024 x 3072 of K = 128 254 -> 260).
+  // whole rows leave together.  Bands / rows, the unfused attention in us:
+  // 40 heads x 3600 (D = 128, 1037 MB) 893 / 860, 2800 (627 MB) 556 / 540, 2560
+  // (524 MB) 447 / 446 (the product alone 143 / 140), 2304 (425 MB) 386 / 385
+  // (115 / 115), 2048 (336 MB) 291 / 293, 1600 (205 MB) 222 / 224; 24 heads x
+  // 4096 (D = 64, 805 MB) 581 / 573.
   g.band = EPI == kEpiRows && 2.0 * (double)batch * (double)g.M * (double)g.N > 512e6 ? 1 : 8;
   const dim3 grid((unsigned)nwork, (unsigned)batch, (unsigned)parts);
-  const int64_t slices = EPI == kEpiPart ? g.part_slices : (g.K + kG2K - 1) / kG2K;
-  if (nwork * batch * parts <= kGmDeepGrid && slices >= kGmDeepSlices)
+  if (mid_lead(g.M, g.N, batch, BM, parts, g.part_slices) == kGmDeep)
     hipLaunchKernelGGL((gemm_mid_kernel<BM, KN, EPI, kGmDeep>), grid, dim3(kG2Threads), 0, st, g);
   else
     hipLaunchKernelGGL((gemm_mid_kernel<BM, KN, EPI, 2>), grid, dim3(kG2Threads), 0, st, g);
@@ -1063,9 +1110,11 @@ static int gemm_run(const uint8_t* a8, const uint8_t* b8, int b_layout, const vo
   if (direct) {
     const bool whole = K % kG2Sub == 0;
     const bool split_ok = item_counter != nullptr && rb.row_scale == nullptr;
-    GemmPlan p = gemm_plan(M, N, K, rb.batch, whole, split_ok);
+    const bool wide_c = reinterpret_cast<uintptr_t>(c) % 16 == 0 && ldc % 8 == 0 &&
+                        (rb.batch == 1 || rb.bsc % 8 == 0);
+    GemmPlan p = gemm_plan(M, N, K, rb.batch, whole, split_ok, wide_c);
     if (p.parts > 1 && workspace_bytes < gemm_workspace_bytes(M, N, p))
-      p = gemm_plan(M, N, K, rb.batch, whole, false);
+      p = gemm_plan(M, N, K, rb.batch, whole, false, wide_c);
     if (p.parts > 1)
       g.part = reinterpret_cast<float*>(reinterpret_cast<char*>(item_counter) +
                                         RP_GEMM_BALANCED_WORKSPACE_BYTES);
@@ -1110,7 +1159,21 @@ extern "C" int rp_fp8_linear_balanced(const uint8_t* a8, const uint8_t* b8, int 
 
 extern "C" size_t rp_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return gemm_workspace_bytes(M, N, gemm_plan(M, N, K, 1, K % kG2Sub == 0, true));
+  // (C's alignment decides nothing where K is split)
+  return gemm_workspace_bytes(M, N, gemm_plan(M, N, K, 1, K % kG2Sub == 0, true, true));
+}
+
+extern "C" int rp_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int may_split,
+                                int* tile_rows, int* k_parts, int* slices_ahead) {
+  if (M <= 0 || N <= 0 || K <= 0 || batch < 1 || !tile_rows || !k_parts || !slices_ahead) {
+    rp_set_error("gemm_plan: bad arguments");
+    return RP_ERR_INVALID_ARGUMENT;
+  }
+  const GemmPlan p = gemm_plan(M, N, K, batch, K % kG2Sub == 0, may_split != 0, N % 8 == 0);
+  *tile_rows = p.bm;
+  *k_parts = p.parts;
+  *slices_ahead = p.bm == kG2Tile ? 2 : mid_lead(M, N, batch, p.bm, p.parts, p.part_slices);
+  return RP_OK;
 }
 
 extern "C" int rp_fp8_gemm_rowwise(const uint8_t* a8, const uint8_t* b8, int b_layout, void* c,
