@@ -357,7 +357,10 @@ int rp_fp8_attn_fwd_balanced(const uint8_t* q8, const uint8_t* k8, const uint8_t
  * 16-byte aligned; the sum of squares runs in the order the header of
  * rp_prologue.hip states.  The workspace holds the amax pass's partial
  * maxima and each row's fp32 inverse norm, which the apply pass reads back
- * (4 bytes per row); it must not be shared by calls that may overlap. */
+ * (4 bytes per row); it must not be shared by calls that may overlap.  The
+ * query's answer is enough for every rope_mode; without tables a per-tensor
+ * call takes less too (a maximum per 16384 elements instead of one per head
+ * and 16384 / D rows). */
 size_t rp_fp8_rmsnorm_quant_workspace_bytes(int64_t B, int64_t H, int64_t S, int64_t D,
                                             int granularity);
 int rp_fp8_rmsnorm_scale_quantize(const void* x, int64_t B, int64_t H, int64_t S, int64_t D,

@@ -754,7 +754,7 @@ int run_norm_qkv(const NormQKV& a, hipStream_t st) {
   return launch_check("rmsnorm_quantize_qkv(apply)");
 }
 
-// Bytes of one tensor's partial maxima and of its rows' inverse norms.
+// Bytes of one tensor's partial maxima, at most, and of its rows' inverse norms.
 struct PSizes {
   size_t partials, rinv;
 };
@@ -897,15 +897,16 @@ extern "C" int rp_fp8_rmsnorm_scale_quantize(const void* x, int64_t B, int64_t H
   int rc = make_pparams(who, x, B, H, S, D, sb, sh, ss, weight, eps, rope_cos, rope_sin,
                         rope_mode, granularity, codes, &p);
   if (rc) return rc;
-  const size_t need = rp_fp8_rmsnorm_quant_workspace_bytes(B, H, S, D, granularity);
+  // what this call writes: without tables fewer maxima than the query's bound
+  const int64_t ngroups = granularity == RP_SCALE_PER_BH ? B * H : 1;
+  const size_t partial_bytes = align256((size_t)(ngroups * p.nbg) * sizeof(uint32_t));
+  const size_t need = partial_bytes + (size_t)(B * H * S) * sizeof(float);
   if (workspace == nullptr || workspace_bytes < need) {
     rp_set_error("%s: workspace of %zu bytes needed, got %zu", who, need, workspace_bytes);
     return RP_ERR_WORKSPACE;
   }
-  const int64_t ngroups = granularity == RP_SCALE_PER_BH ? B * H : 1;
   uint32_t* partial = static_cast<uint32_t*>(workspace);
-  const size_t partial_bytes = (size_t)(ngroups * p.nbg) * sizeof(uint32_t);
-  p.rinv = reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(partial_bytes));
+  p.rinv = reinterpret_cast<float*>(static_cast<char*>(workspace) + partial_bytes);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int per_bh = granularity == RP_SCALE_PER_BH;
   return with_layout(D, rope_mode, [&](auto d_c, auto r_c) {
@@ -960,14 +961,20 @@ extern "C" int rp_fp8_rmsnorm_scale_quantize_qkv(
     rp_set_error("%s: vt8 must be 16-byte aligned", who);
     return RP_ERR_UNSUPPORTED;
   }
-  const size_t need = rp_fp8_rmsnorm_quant_qkv_workspace_bytes(B, H, Sq, Skv, D, granularity);
+  // the regions of the workspace (as the query counts them, but with this
+  // call's own number of maxima)
+  const int64_t ngroups = granularity == RP_SCALE_PER_BH ? B * H : 1;
+  const size_t o_pk = align256((size_t)(ngroups * a.q.nbg) * sizeof(uint32_t));
+  const size_t o_pv = o_pk + align256((size_t)(ngroups * a.k.nbg) * sizeof(uint32_t));
+  const size_t o_rq = o_pv + align256(pv.ws_bytes);
+  const size_t o_rk = o_rq + align256((size_t)(B * H * Sq) * sizeof(float));
+  const size_t need = o_rk + (size_t)(B * H * Skv) * sizeof(float);
   if (workspace == nullptr || workspace_bytes < need ||
       reinterpret_cast<uintptr_t>(workspace) % 256 != 0) {
     rp_set_error("%s: workspace of %zu bytes (256-byte aligned) needed, got %zu", who, need,
                  workspace_bytes);
     return RP_ERR_WORKSPACE;
   }
-  const int64_t ngroups = granularity == RP_SCALE_PER_BH ? B * H : 1;
   a.v = pv.p;
   a.vt = QParams{};
   a.vt.x = static_cast<const uint16_t*>(v);
@@ -988,16 +995,11 @@ extern "C" int rp_fp8_rmsnorm_scale_quantize_qkv(
     return RP_ERR_UNSUPPORTED;
   }
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  size_t off = 0;
-  a.pq = reinterpret_cast<uint32_t*>(ws + off);
-  off += align256((size_t)(ngroups * a.q.nbg) * sizeof(uint32_t));
-  a.pk = reinterpret_cast<uint32_t*>(ws + off);
-  off += align256((size_t)(ngroups * a.k.nbg) * sizeof(uint32_t));
-  a.pv = reinterpret_cast<uint32_t*>(ws + off);
-  off += align256(pv.ws_bytes);
-  a.q.rinv = reinterpret_cast<float*>(ws + off);
-  off += align256((size_t)(B * H * Sq) * sizeof(float));
-  a.k.rinv = reinterpret_cast<float*>(ws + off);
+  a.pq = reinterpret_cast<uint32_t*>(ws);
+  a.pk = reinterpret_cast<uint32_t*>(ws + o_pk);
+  a.pv = reinterpret_cast<uint32_t*>(ws + o_pv);
+  a.q.rinv = reinterpret_cast<float*>(ws + o_rq);
+  a.k.rinv = reinterpret_cast<float*>(ws + o_rk);
   a.dequant = dequant_out;
   a.q8 = q8;
   a.k8 = k8;

@@ -251,3 +251,50 @@ def test_rotary_few_ranges_equal_single_heads(gpu: torch.device, B: int, H: int,
             d, c = ops.rmsnorm_scale_quantize(x[b:b + 1, h:h + 1], w, 1e-6, t, rope, "bh")
             assert torch.equal(dq.view(B, H)[b, h], d[0])
             assert torch.equal(codes[b, h].view(torch.uint8), c[0, 0].view(torch.uint8))
+
+
+@pytest.mark.parametrize("qkv", [False, True])
+def test_per_tensor_call_without_tables_takes_its_own_workspace(gpu: torch.device,
+                                                                qkv: bool) -> None:
+    """Without tables a per-tensor call writes a maximum per 16384 elements, and
+    a workspace of that many and the inverse norms is enough (the query's
+    answer covers the rotary calls too); four bytes less are refused."""
+    from repercep_runtime_amd import _capi as C
+    B, H, S, D = 4, 64, 10, 128
+    L, g = C.lib(), C.RP_SCALE_PER_TENSOR
+    q, k, v = (_x(i, (B, H, S, D), 2.0).to(gpu) for i in range(3))
+    rows, up = B * H * S, lambda n: -(-n // 256) * 256
+    part = up(4 * -(-rows * D // 16384))
+    st = (H * S * D, S * D, D)
+    codes = torch.zeros((3, rows * D), dtype=torch.uint8, device=gpu)
+    vt = torch.zeros((B, H, D, 128), dtype=torch.uint8, device=gpu)
+    dq = torch.zeros(3, device=gpu)
+    if qkv:
+        size, most = 3 * part + up(4 * rows) + 4 * rows, \
+            L.rp_fp8_rmsnorm_quant_qkv_workspace_bytes(B, H, S, S, D, g)
+    else:
+        size, most = part + 4 * rows, L.rp_fp8_rmsnorm_quant_workspace_bytes(B, H, S, D, g)
+    assert size < most
+    ws = torch.full((size + 1024,), 0xA5, dtype=torch.uint8, device=gpu)
+
+    def call(n: int) -> int:
+        if qkv:
+            return L.rp_fp8_rmsnorm_scale_quantize_qkv(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), B, H, S, S, D, *st, *st, *st, None,
+                None, 1e-6, None, None, None, None, 0, g, dq.data_ptr(), codes[0].data_ptr(),
+                codes[1].data_ptr(), vt.data_ptr(), 128, ws.data_ptr(), n, ops._stream(q))
+        return L.rp_fp8_rmsnorm_scale_quantize(
+            q.data_ptr(), B, H, S, D, *st, None, 1e-6, None, None, 0, g, dq.data_ptr(),
+            codes[0].data_ptr(), ws.data_ptr(), n, ops._stream(q))
+
+    assert call(size - 4) == 3
+    assert call(size) == 0
+    torch.cuda.synchronize()
+    assert bool((ws[size:] == 0xA5).all())
+    for i, x in enumerate((q, k) if qkv else (q,)):
+        d, c = ops.rmsnorm_scale_quantize(x, None, 1e-6, None, "half", "tensor")
+        assert torch.equal(dq[i], d[0])
+        assert torch.equal(codes[i], c.view(torch.uint8).reshape(-1))
+    if qkv:
+        d, c = ops.scale_quantize(v, "tensor", "bhds")
+        assert torch.equal(dq[2], d[0]) and torch.equal(vt, c.view(torch.uint8).view_as(vt))
