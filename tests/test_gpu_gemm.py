@@ -1,7 +1,10 @@
 """GPU parity of the FP8 scaled GEMM.
 
-Shapes with K a multiple of 64 run the large-tile kernel (one to nine 64-deep
-K slices, ragged M and N); K = 48 and K = 16 run the general kernel.
+Which kernel a shape runs on is rp_fp8_gemm_plan's (tests/test_gemm_plan.py):
+small products take the medium tiles, whatever their K (tests/
+test_gpu_gemm_mid.py), the large ones below the 256 x 256 tiles, and a (K, N) B
+whose N is no multiple of 16, or strides past 32-bit tile offsets, the general
+kernel.
 
 Reference: kernels/hip/fp8_attn/fp8_gemm.hip:79-179 and its known-answer
 tests tests/test_mfma_fragment_layout.py:262-315 (restated here for the
@@ -20,6 +23,7 @@ from repercep_runtime_amd import ops
 from repercep_runtime_amd.workloads import C4, gemm_inputs
 from oracle.quant import DECODE
 from tests._helpers import bf16_bits, bf16_to_f32, bf16_ulp, codes_np, err_stats
+from tests.test_gemm_plan import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -104,13 +108,14 @@ def test_random_vs_oracle(gpu: torch.device, mnk: tuple[int, int, int]) -> None:
     ((64, 256, 64), 0),        # one 64-deep K slice
     ((513, 272, 192), 16),     # N % 256 == 16: one granule in the last tile
     ((100, 100, 4160), 0),     # N % 16 != 0: the general kernel's byte gathers
-    ((33, 12, 48), 4),         # K % 64 != 0, odd ldb: the general kernel
+    ((33, 12, 48), 4),         # and K % 64 != 0, odd ldb
 ])
 def test_row_major_b_vs_oracle(gpu: torch.device, mnk: tuple[int, int, int],
                                ldb_pad: int, monkeypatch: pytest.MonkeyPatch) -> None:
     """B given as the reference passes it, (K, N) row-major (rp_fp8_gemm with
-    RP_B_KN): no transpose pass runs, and the result is the (N, K) path's
-    bit for bit and within one rounding of the exact sum."""
+    RP_B_KN): no transpose pass runs, and the result is within one rounding of
+    the exact sum, and the (N, K) path's bit for bit where both run the same
+    kernel (the general one, for N % 16, sums in another order)."""
     M, N, K = mnk
     g = torch.Generator().manual_seed(7 * M + N + K)
     a8 = torch.randn(M, K, generator=g).mul(30).to(torch.float8_e4m3fn)
@@ -122,11 +127,13 @@ def test_row_major_b_vs_oracle(gpu: torch.device, mnk: tuple[int, int, int],
     monkeypatch.setattr(ops, "transpose_fp8", lambda *_a, **_k: pytest.fail("transpose pass ran"))
     got = ops.fp8_gemm(a8.to(gpu), bview, sa, sb)
     nk = ops.fp8_gemm(a8.to(gpu), b8.t().contiguous().to(gpu), sa, sb, b_transposed=True)
-    assert torch.equal(got, nk), f"max diff {(got.float() - nk.float()).abs().max().item()}"
+    if N % 16 == 0:
+        assert torch.equal(got, nk), f"max diff {(got.float() - nk.float()).abs().max().item()}"
     bt = np.ascontiguousarray(codes_np(b8).T)
     ref = native.gemm_rows(codes_np(a8), bt, sa, sb, np.arange(M))
-    _assert_one_rounding_apart(bf16_to_f32(bf16_bits(got)), bf16_to_f32(ref), codes_np(a8),
-                               bt, sa * sb)
+    for c in (got, nk):
+        _assert_one_rounding_apart(bf16_to_f32(bf16_bits(c)), bf16_to_f32(ref), codes_np(a8),
+                                   bt, sa * sb)
 
 
 def test_weight_with_unaligned_n_and_k(gpu: torch.device) -> None:
@@ -147,12 +154,13 @@ def test_weight_with_unaligned_n_and_k(gpu: torch.device) -> None:
     assert float(ws_ref[0]) == float(sw.item())
     assert np.array_equal(codes_np(w8), w8_ref) and np.array_equal(codes_np(wt8), w8_ref.T)
     c_nk = ops.fp8_gemm(a8, wt8, sa, sw, b_transposed=True)
-    c_kn = ops.fp8_gemm(a8, w8, sa, sw)
-    assert torch.equal(c_nk, c_kn)
+    c_kn = ops.fp8_gemm(a8, w8, sa, sw)     # N % 16: the general kernel; the other splits K
     ref = native.gemm_rows(codes_np(a8), np.ascontiguousarray(w8_ref.T), float(sa.item()),
                            float(sw.item()), np.arange(M))
-    _assert_one_rounding_apart(bf16_to_f32(bf16_bits(c_nk)), bf16_to_f32(ref), codes_np(a8),
-                               np.ascontiguousarray(w8_ref.T), float(sa.item()) * float(sw.item()))
+    for c in (c_nk, c_kn):
+        _assert_one_rounding_apart(bf16_to_f32(bf16_bits(c)), bf16_to_f32(ref), codes_np(a8),
+                                   np.ascontiguousarray(w8_ref.T),
+                                   float(sa.item()) * float(sw.item()))
 
 
 @pytest.mark.parametrize("mnk", [(64, 64, 256), (300, 200, 512), (5, 4, 16)])
@@ -179,9 +187,9 @@ def test_bias_epilogue_small_integers_exact(gpu: torch.device, mnk: tuple[int, i
 @pytest.mark.parametrize("mnk", [(257, 520, 384), (1000, 64, 512), (600, 520, 192),
                                  (513, 260, 48)])
 def test_bias_epilogue_vs_oracle(gpu: torch.device, mnk: tuple[int, int, int]) -> None:
-    """Both GEMM kernels (256x256 tiles when K % 64 == 0, the 256x128 fallback
-    otherwise) with a bias: every output within one rounding of
-    exact * scale + bias, and with a zero bias bit-identical to rp_fp8_gemm."""
+    """A bias on small products (the medium tiles), K a multiple of 64 and not:
+    every output within one rounding of exact * scale + bias, and with a zero
+    bias bit-identical to the product without one."""
     M, N, K = mnk
     g = torch.Generator().manual_seed(3 * M + N + K)
     a8 = torch.randn(M, K, generator=g).mul(30).to(torch.float8_e4m3fn)
@@ -287,20 +295,21 @@ def _linear_static(a8, b8, layout, bias, out, M, N, K, sa, sb):
 
 
 @pytest.mark.parametrize("M,N,K,layout,with_bias", [
-    (300, 272, 128, "kn", False),     # 4 tiles: shares of 0 and 1 tiles, nothing to pool
-    (2148, 1280, 128, "kn", True),    # 45 tiles: shares of 6 and 5, every tile pooled
-    (2560, 2304, 192, "nk", True),    # 90 tiles: shares of 12 and 11, every tile pooled
-    (C4.M, C4.N, 512, "kn", False),   # the C4 grid (15,984 tiles): 64 pooled per share
-    (C4.M, C4.N, 512, "nk", True),
+    (3840, 3600, 1088, "kn", False),   # 225 tiles: shares of 29 and 28, every tile pooled
+    (3840, 3600, 1088, "nk", True),
+    (4090, 3600, 1216, "kn", True),    # 240 tiles: equal shares, ragged M
+    (C4.M, C4.N, 1152, "kn", False),   # the C4 grid (15,984 tiles): 64 pooled per share
+    (C4.M, C4.N, 1152, "nk", True),
 ])
 def test_balanced_gemm_equals_static_tiles(gpu: torch.device, M: int, N: int, K: int,
                                            layout: str, with_bias: bool) -> None:
     """rp_fp8_linear_balanced (the op's launch: the last tiles of every XCD's
     share handed out through a counter) writes rp_fp8_linear's bits, on grids
-    too small to pool, where every tile is pooled and the XCD shares differ by
-    one tile, and on C4's grid; two calls in a row reuse the workspace (the call zeroes its
-    counter itself)."""
+    of the large tiles so small that every tile is pooled, with XCD shares
+    that differ by one tile and that do not, and on C4's grid; two calls in a
+    row reuse the workspace (the call zeroes its counter itself)."""
     from repercep_runtime_amd import _capi as C
+    assert plan(M, N, K)[:2] == plan(M, N, K, 1, 0)[:2] == (256, 1)
     g = torch.Generator(device=gpu).manual_seed(M + N + K)
     a8 = torch.randint(0, 126, (M, K), generator=g, device=gpu, dtype=torch.uint8)
     b8 = torch.randint(0, 126, (K, N) if layout == "kn" else (N, K), generator=g, device=gpu,
@@ -317,3 +326,93 @@ def test_balanced_gemm_equals_static_tiles(gpu: torch.device, M: int, N: int, K:
             out.data_ptr(), M, N, K, a8.stride(0), b8.stride(0), out.stride(0), 0.01, 0.02, None,
             None, ws.data_ptr(), ws.numel(), ops._stream(a8)), "rp_fp8_linear_balanced")
         assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+ROWS = np.array([0, 1, 31, 255, 256, 1023, 4095, 4089])   # of 4090: tile edges, the last tile
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("N,K,layout,pad,off", [
+    (3596, 1088, "nk", 0, 0),      # ragged N, half last K slice, C rows on 8 bytes
+    (3600, 1088, "kn", 0, 0),      # ragged granules of a (K, N) B
+    (3600, 1152, "nk", 12, 4),     # strided C, 8 bytes off alignment, whole slices
+    (3600, 1152, "kn", 8, 8),      # strided C on 16 bytes
+])
+def test_large_tiles_vs_exact(gpu: torch.device, N: int, K: int, layout: str, pad: int, off: int,
+                              bias: bool) -> None:
+    """The 256 x 256 kernel at its edges: ragged M and N, K % 128 == 64, both
+    layouts, bias, strided and unaligned C -- sampled rows against the exact
+    product, the padding around C untouched."""
+    M = 4090
+    assert plan(M, N, K)[:2] == (256, 1)
+    rows = np.minimum(ROWS, M - 1)
+    g = torch.Generator().manual_seed(N + K + pad)
+    a8 = torch.randn(M, K, generator=g).mul(30).to(torch.float8_e4m3fn)
+    bt8 = torch.randn(N, K, generator=g).mul(30).to(torch.float8_e4m3fn)
+    b = torch.randn(N, generator=g).mul(50).to(torch.bfloat16) if bias else None
+    bg = bt8.to(gpu)
+    if layout == "kn":
+        bg = bg.view(torch.uint8).t().contiguous().view(torch.float8_e4m3fn)
+    wide = torch.full((M, off + N + pad), 7.0, dtype=torch.bfloat16, device=gpu)
+    got = ops.fp8_gemm(a8.to(gpu), bg, 0.013, 0.0071, b_transposed=layout == "nk",
+                       bias=b.to(gpu) if bias else None, out=wide[:, off:off + N])
+    _assert_one_rounding_apart(bf16_to_f32(bf16_bits(got[torch.from_numpy(rows).to(gpu)])), None,
+                               codes_np(a8)[rows], codes_np(bt8), 0.013 * 0.0071,
+                               b.float().numpy().astype(np.float64) if bias else None)
+    assert not bool(torch.isnan(got).any())
+    rest = torch.cat([wide[:, :off], wide[:, off + N:]], dim=1)
+    assert bool((rest == 7.0).all())
+
+
+def test_large_tiles_row_scaled_batch(gpu: torch.device) -> None:
+    """The 256 x 256 kernel's row-scaled epilogue over a batch, ragged in M, N
+    and K: small integers and powers of two, exact."""
+    Z, M, N, K = 2, 4090, 3596, 1088
+    assert plan(M, N, K, Z, 0)[0] == 256
+    g = torch.Generator(device=gpu).manual_seed(5)
+    a = torch.randint(-2, 3, (Z, M, K), generator=g, device=gpu).float()
+    b = torch.randint(-2, 3, (Z, N, K), generator=g, device=gpu).float()
+    sa = 2.0 ** torch.randint(-4, 4, (Z, M), generator=g, device=gpu).float()
+    sb = 2.0 ** torch.randint(-4, 4, (Z, N), generator=g, device=gpu).float()
+    got = ops.gemm_rowwise(a.to(torch.float8_e4m3fn), b.to(torch.float8_e4m3fn), sa, sb)
+    for z in range(Z):
+        want = ((a[z] @ b[z].t()) * sa[z, :, None] * sb[z, None, :]).to(torch.bfloat16)
+        assert torch.equal(got[z], want)
+
+
+@pytest.mark.parametrize("far", ["a", "b", "rows"])
+def test_strides_past_32_bit_tile_offsets(gpu: torch.device, far: str) -> None:
+    """Row strides of 2^24 bytes (256 rows of them reach 2^32) run the general
+    kernel, on an (N, K) B, with a bias, and with row scales."""
+    M, N, K, ld = 5, 12, 208, 1 << 24
+    g = torch.Generator().manual_seed(17)
+    a8 = torch.randn(M, K, generator=g).mul(30).to(torch.float8_e4m3fn)
+    bt8 = torch.randn(N, K, generator=g).mul(30).to(torch.float8_e4m3fn)
+
+    def strided(x: torch.Tensor) -> torch.Tensor:
+        flat = torch.zeros(x.shape[0] * ld, dtype=torch.uint8, device=gpu)
+        v = flat.as_strided((x.shape[0], K), (ld, 1))
+        v.copy_(x.view(torch.uint8))
+        return v
+
+    if far == "rows":
+        sa, sb = (2.0 ** torch.randint(-4, 4, (n,), generator=g).float() for n in (M, N))
+        ai = torch.randint(-2, 3, (M, K), generator=g).float()
+        bi = torch.randint(-2, 3, (N, K), generator=g).float()
+        from repercep_runtime_amd import _capi as C
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=gpu)
+        av, bv = strided(ai.to(torch.float8_e4m3fn)), bi.to(torch.float8_e4m3fn).to(gpu)
+        sag, sbg = sa.to(gpu), sb.to(gpu)
+        C.check(C.lib().rp_fp8_gemm_rowwise(
+            av.data_ptr(), bv.data_ptr(), C.RP_B_NK, out.data_ptr(), M, N, K, ld, K, N,
+            sag.data_ptr(), sbg.data_ptr(), 1, 0, 0, 0, 0, 0, ops._stream(out)),
+            "rp_fp8_gemm_rowwise")
+        want = ((ai @ bi.t()) * sa[:, None] * sb[None, :]).to(torch.bfloat16)
+        assert torch.equal(out.cpu(), want)
+        return
+    bias = torch.randn(N, generator=g).mul(50).to(torch.bfloat16)
+    got = ops.fp8_gemm(strided(a8) if far == "a" else a8.to(gpu),
+                       strided(bt8) if far == "b" else bt8.to(gpu), 0.013, 0.0071,
+                       b_transposed=True, bias=bias.to(gpu))
+    _assert_one_rounding_apart(bf16_to_f32(bf16_bits(got)), None, codes_np(a8), codes_np(bt8),
+                               0.013 * 0.0071, bias.float().numpy().astype(np.float64))

@@ -10,6 +10,7 @@ import torch
 
 from repercep_runtime_amd import ops
 from repercep_runtime_amd.workloads import C1, C5, attn_inputs
+from tests.test_gemm_plan import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -67,7 +68,8 @@ def test_captured_balanced_gemm_replays_match_eager(gpu: torch.device) -> None:
     call, tiles handed out through it) captured with its workspace from the
     capture's pool: every replay, with new operands, equals an eager call bit
     for bit."""
-    M, N, K = 2148, 1280, 256    # 45 tiles: every tile goes through the counter
+    M, N, K = 3840, 3600, 1088    # 225 large tiles: every tile goes through the counter
+    assert plan(M, N, K)[:2] == (256, 1)
     g = torch.Generator(device=gpu).manual_seed(13)
     a8 = torch.randint(0, 126, (M, K), generator=g, device=gpu, dtype=torch.uint8)
     b8 = torch.randint(0, 126, (K, N), generator=g, device=gpu, dtype=torch.uint8)
