@@ -61,6 +61,8 @@
 
 #include "rp_common.h"
 
+#include <math.h>
+
 #include <utility>
 
 namespace rp {
@@ -1250,6 +1252,25 @@ struct TailPlan {
   int main_blocks;   // query blocks per head run unsplit
   int splits;        // key splits of the remaining blocks (1: a plain launch)
 };
+// What the tail of a launch costs, in key tiles: rounds of workgroups of
+// n_kb / sp tiles and their fixed cost each, a partial round of split ones
+// between `first` of a round and a whole one (the pooled unsplit items even
+// its end out), and for a split the merge launch and the parts, 128 KiB each,
+// written and read.  Fits per head dim, whose tiles take 1.2, 2 and 2.7 us at
+// D = 64, 128 and 256, to 561 shapes (8-80 heads of 1100-59000 rows) timed
+// unsplit and split 2, 4 and 8 ways.  The plan is behind the best of the four
+// by 0.06%, 0.29% and 0.27% on average and 1.2%, 2.4% and 2.8% at most.
+// Rounds alone, without the fixed costs and the parts, were 4.4% behind on
+// average and 82% at most (80 heads x 3538 at D = 256 split four ways 1256 us,
+// unsplit 946; 32 x 14080 at D = 128 eight ways 1.86 ms, unsplit 1.75); one set
+// of constants for all head dims 0.43% and 5.3% (12 x 17707 at D = 256 unsplit
+// 2784 us, eight ways 2688).  A split changes which running maximum P is
+// rounded under, so the same rows differ by ~1% between two plans; unsplit is
+// the one-range algorithm itself (error of the tail rows against 64 bits, N(0, 1)
+// inputs, 32 x 14080 at D = 128: unsplit 0.0526, two to eight ways 0.0525-0.0521).
+struct TailCost {
+  double fixed, fixed_split, merge, part, first;
+};
 inline TailPlan tail_plan(int B, int H, int Sq, int Skv, int D, int mask, int cus) {
   const int nq = (Sq + kBlockM - 1) / kBlockM;
   TailPlan t{nq, 1};
@@ -1266,15 +1287,16 @@ inline TailPlan tail_plan(int B, int H, int Sq, int Skv, int D, int mask, int cu
   // the unsplit workgroups spread evenly over the 8 XCDs
   if (m == nq || m == 0 || (per_block * m) % 8 != 0) return t;
   const int64_t tail = per_block * (nq - m);
-  // In key tiles (~2 us): rounds of workgroups of n_kb / sp tiles and the
-  // fixed cost each, and for a split the merge launch (~5 us) and the parts,
-  // 128 KiB each, written and read at ~4 TB/s.  (Without the fixed cost and
-  // the parts' bytes the plan split 224 of (1, 32, 14080, 14080, 128)'s 1760
-  // workgroups eight ways: the call took 1.86 ms, 1.75 unsplit.)
+  const TailCost tc = D == 256 ? TailCost{2.0, 3.0, 2.5, 0.016, 0.6}
+                      : D == 128 ? TailCost{7.0, 7.0, 5.0, 0.020, 0.8}
+                                 : TailCost{2.0, 2.0, 5.0, 0.020, 0.9};
   auto cost_of = [&](int sp) {
-    const double parts = (double)tail * sp;
-    return (double)((tail * sp + cus - 1) / cus) * ((double)n_kb / sp + (double)kFixedTiles) +
-           (sp > 1 ? 2.5 + parts * 0.033 : 0.0);
+    const double parts = (double)tail * sp, rounds = parts / (double)cus;
+    if (sp == 1) return ceil(rounds) * ((double)n_kb + tc.fixed);
+    const double part_round = rounds - floor(rounds);
+    return (floor(rounds) + (part_round > 0.0 ? tc.first + (1.0 - tc.first) * part_round : 0.0)) *
+               ((double)n_kb / sp + tc.fixed_split) +
+           tc.merge + parts * tc.part;
   };
   double best = cost_of(1);
   int best_s = 1;
