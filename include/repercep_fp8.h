@@ -114,8 +114,8 @@ int rp_fp8_scale_quantize(const void* x, int x_dtype, int64_t B, int64_t H, int6
 /* Q, K and V of one attention call in one call: the scales and codes of
  * rp_fp8_scale_quantize for q and k ((B, H, S, D) codes) and for v (V^T,
  * (B, H, D, ldv)), from four kernel launches (amax of all three, their
- * scales, q and k codes, V^T codes) instead of nine -- launches bound small
- * calls.  dequant_out: float[3 * G], G = B*H (RP_SCALE_PER_BH) or 1, in the
+ * scales, q and k codes, V^T codes) instead of nine, or two or one where the
+ * groups are small -- launches bound small calls.  dequant_out: float[3 * G], G = B*H (RP_SCALE_PER_BH) or 1, in the
  * order q, k, v.  workspace: rp_fp8_quant_qkv_workspace_bytes, 256-byte
  * aligned.  Replaces the three _per_bh_scale + _quantize pairs at
  * kernels/triton_kernels/fp8_flash_attn.py:522-528 with one host call.
@@ -412,8 +412,10 @@ int rp_fp8_rmsnorm_scale_quantize_qkv(const void* q, const void* k, const void* 
  * they are used instead of the host values, avoiding a device->host read.
  * K, lda multiples of 16; N, ldc multiples of 4; a8 16-byte aligned, c
  * 8-byte aligned; RP_B_NK also needs ldb % 16 == 0 and b8 16-byte aligned.
- * Fastest path: K % 64 == 0 (and for RP_B_KN, N and ldb multiples of 16,
- * b8 16-byte aligned); other shapes run a general kernel. */
+ * Any such K runs the direct-to-LDS kernels (for RP_B_KN, with N and ldb
+ * multiples of 16 and b8 16-byte aligned), grids that fill the GPU fastest
+ * with K % 64 == 0; other RP_B_KN operands and row strides past 2^24 run a
+ * general kernel. */
 #define RP_B_NK 0
 #define RP_B_KN 1
 int rp_fp8_gemm(const uint8_t* a8, const uint8_t* b8, int b_layout, void* c,

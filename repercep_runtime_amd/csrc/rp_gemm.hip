@@ -852,7 +852,9 @@ struct GemmPlan {
 //   the medium tiles' is too low.
 // * C rows off 16 bytes, past the 256 MB cache: the medium tiles' stores lose
 //   (40 x 2500 x 2500 of K = 256 / 512 1.06 / 1.14).
-// Of the 429 a handful take the slower form, by 5% at the most.
+// Of the 429 a handful take the slower form, by 5% at the most (in another
+// sweep 8192 x 3072 x 3072, (K, N) weights from HBM, by 7%: 81.7 against 76.5
+// us; with warm weights 70.0 against 76.7).
 inline bool medium_pays(int64_t M, int64_t N, int64_t K, int64_t batch, double t128, double t256,
                         bool wide_c) {
   const double ns = (double)((K + kG2K - 1) / kG2K);
@@ -881,10 +883,11 @@ inline bool medium_pays(int64_t M, int64_t N, int64_t K, int64_t batch, double t
 //   launch, ~5.5.
 // These constants are fits to the two-ahead ring with (N, K) weights used
 // again and again, over M 16 .. 16384 of seven projections.  The four-ahead
-// ring, (K, N) weights and weights from HBM are not modelled: over the nine
-// projections the choice is within 4% of the best form in four products of
-// five, and at worst 1.36 times it (700 x 1536 x 8960 with weights from HBM,
-// 32.6 against 23.9 us).
+// ring, (K, N) weights and weights from HBM are not modelled: over 216 products
+// of the nine projections, M 16 .. 8192, the choice is more than 4% behind the
+// best form in 30 with warm weights and in 38 with weights from HBM, by 21%
+// and 35% at worst (512 x 5120 x 13824 in (K, N) 56.8 against 46.9 us; 700 x
+// 1536 x 8960 32.2 against 23.8).
 // A row-scaled (batched) product is never split; nor one whose caller brings
 // no workspace (may_split).  The CU count is the MI355X's.
 inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool whole,

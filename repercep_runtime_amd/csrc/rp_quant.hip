@@ -349,18 +349,20 @@ int launch_amax(const Plan& pl, uint32_t* partial, hipStream_t st) {
 }
 
 // Whether a Q/K/V call of `groups` groups of up to `elems` elements and
-// `tiles` V^T tiles each, which fit quant_group_kernel, runs in its one launch.  GPU time in us, two launches
-// (amax_multi, apply_fold_multi) / one (contiguous Q, K, V; groups x elements):
+// `tiles` V^T tiles each, which fit quant_group_kernel, runs in its one
+// launch.  GPU time in us, two launches (amax_multi, apply_fold_multi) / one
+// (contiguous Q, K, V; groups x elements):
 //    8 x 1024    6.7 / 7.0       8 x 32768   7.8 / 7.4      640 x 1024   10.7 / 21.7
 //   40 x 8192    8.5 / 7.2      80 x 32768  11.9 / 8.4      640 x 8192   18.3 / 23.6
 //    8 x 65536   7.9 / 9.8     320 x 32768  29.0 / 20.5    2560 x 8192   58.6 / 74.2
 //   16 x 65536   9.7 / 10.1     40 x 65536  12.3 / 11.2    2560 x 16384   102 / 91
 // One CU per group is slower where it has a whole group of 65536 to convert
-// (or eight V^T tiles, full or not) and the others wait, and where so small a group leaves most of its 1024
-// threads idle that the groups queue.  An eager call is bound by its launches:
-// it takes 25-26 us in two and 22-23 in one (8 to 160 groups of any size), so
-// there the saved launch counts, up to as many workgroups as run at once (two
-// per CU); a captured graph replays without the host, so its GPU time counts.
+// (or eight V^T tiles, full or not) and the others wait, and where so small a
+// group leaves most of its 1024 threads idle that the groups queue.  An eager
+// call is bound by its launches: it takes 25-26 us in two and 22-23 in one (8
+// to 160 groups of any size), so there the saved launch counts, up to as many
+// workgroups as run at once (two per CU); a captured graph replays without the
+// host, so its GPU time counts.
 bool one_launch_pays(int64_t groups, int64_t elems, int64_t tiles, bool capturing) {
   const bool threads_busy = elems >= 16384 || (elems >= 8192 && groups <= 170);
   const bool cus_busy = max(elems, tiles * 128 * 64) <= 32768 || groups >= 32;

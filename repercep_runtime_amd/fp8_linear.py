@@ -14,7 +14,10 @@ weight as OCP e4m3fn codes with one per-tensor scale and runs the FP8 GEMM:
              attention quantizer's arithmetic), then
              y = bf16(fp32(x8 . W8^T) * sa * sw + bias)   [rp_fp8_linear: the
              product and the bias sum each rounded to fp32, as a bf16
-             nn.Linear's fp32 epilogue; rp_fp8_gemm without a bias]
+             nn.Linear's fp32 epilogue; rp_fp8_gemm without a bias].  The
+             order of the fp32 sums follows from the layer and the number of
+             rows (``ops.fp8_gemm``), so a row's last bit may depend on how
+             many rows x has, as sa depends on all of them
 
 Same members as the reference's module: ``qweight``, ``scale`` (buffers, so
 ``.to()`` and state dicts work), ``bias`` (a Parameter or None),

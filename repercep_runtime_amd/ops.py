@@ -204,8 +204,8 @@ def scale_quantize_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                        ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor,
                                   torch.Tensor, torch.Tensor]:
     """(q_scale, q8, k_scale, k8, v_scale, vt8) of one attention call from one
-    library call (rp_fp8_scale_quantize_qkv: four kernel launches instead of
-    nine) into one device allocation: the same scales and codes as three
+    library call (rp_fp8_scale_quantize_qkv: one, two or four kernel launches
+    instead of nine) into one device allocation: the same scales and codes as three
     ``scale_quantize`` calls (V transposed, "bhds"), with a fraction of the
     host work, which is what bounds small calls.  (B, H, S, D) inputs, bf16 or
     fp16, any strides with a contiguous head dim; K and V share their shape."""
@@ -835,6 +835,11 @@ def fp8_gemm(a8: torch.Tensor, b8: torch.Tensor, a_scale: float | torch.Tensor,
     tensors (read on the device, no host sync).  ``bias`` (bf16 [N]) is added
     to the fp32 product before the bf16 rounding (``rp_fp8_linear``, an
     nn.Linear epilogue; the reference GEMM has none).
+
+    The fp32 sums run in an order that (M, N, K) fix: a product whose few rows
+    would leave most CUs idle sums parts of K side by side and adds them in
+    order.  So equal calls give equal bits, but a row's last bit may depend on
+    how many rows the call has.
     """
     _check_cuda("a8", a8)
     _on_device_of(a8, b8=b8, out=out, bias=bias,
