@@ -415,12 +415,19 @@ constexpr int kRopeMaxHeads = 16;   // LDS words for a block's heads
 constexpr int kRopeHeads = 8;       // heads per block
 // Fewer heads per block, down to two, below this many blocks (per tensor): at
 // (1, 40, 16384, 128) 1024 and 256 take 0.264 and 0.267 ms, 3000 0.284 ms.
-// Calls of 64 to 2048 positions reach the floor of two heads and are no
-// slower with it than with a head per block and chunk per thread (Q, K and V,
-// us: (1, 40, 512, 128) 27.4 / 22.4, (2, 16, 256, 64) 20.8 / 19.8,
-// (8, 32, 1024, 128) 149 / 113); of up to 8 positions they are, by 1.0-1.9 us
-// of GPU time (8.4 / 9.7 at (1, 40, 1, 64)), which eager launches hide.
 constexpr int64_t kRopeMinBlocks = 1024;
+// One head per block while that makes at most this many blocks (per tensor):
+// the chain of one row's steps is such a call's time, and two heads side by
+// side only lengthen it.  A head per block and chunk per thread (before the
+// tables were kept in registers) / two heads / one, Q, K and V from a graph,
+// us: (1, 40, 1, 128) 8.6 / 9.8 / 8.7; (8, 32, 1, 128) 9.6 / 11.5 / 9.9;
+// (8, 32, 32, 64) 10.8 / 12.0 / 10.5; (1, 40, 512, 128) 33.1 / 22.7 / 21.0;
+// 256 blocks, (4, 32, 256, 128) 35.1 / 28.7 / 23.6; 320, (1, 32, 1280, 128)
+// 40.1 / 29.9 / 29.6; 360, (1, 40, 1152, 128) 43.4 / 30.8 / 33.2; 512,
+// (8, 32, 256, 128) 46.5 / 33.0 / 46.6.  More blocks of a few positions each
+// remain slower than they were: (16, 32, 1, 128) 11.8 / 12.7 / 13.9, (32, 32, 4,
+// 128) 18.0 / 19.4 / 22.2.
+constexpr int64_t kRopeSingleBlocks = 320;
 
 // two fp32 -> their nearest-even bf16 values as fp32 (one v_cvt_pk_bf16_f32)
 // and the packed pair
@@ -494,8 +501,9 @@ __device__ __forceinline__ uint32_t rope_row(float (&x)[16], float r, bool has_w
 // (With every range on one XCD, a call of fewer than eight ranges ran on as
 // many XCDs, and nine ranges took two turns on one of them.  Q, K and V in a
 // call, us: (8, 32, 64, 128) 33.1 -> 18.8; (8, 32, 512, 64) 66.1 -> 37.5;
-// (1, 40, 512, 128) 27.8 -> 22.4; whole groups of eight the same.  With a
-// head per block, before the tables were kept in registers: 20.8, 47.6, 27.4.)
+// (1, 40, 512, 128) 27.8 -> 22.4, with two heads per block; whole groups of
+// eight the same.  With a head per block, before the tables were kept in
+// registers: 20.8, 47.6, 27.4.)
 struct RopeBlock {
   uint32_t range, chunk;
 };
@@ -507,16 +515,16 @@ __host__ __device__ inline RopeBlock rope_block(uint32_t b, uint32_t ranges, uin
   return {(ranges & ~7u) + L / chunks, L % chunks};
 }
 
-// Block b of one tensor.  APPLY: codes under the given scales; else the
-// partial maxima, one per (head, row range).
-template <int D, int ROPE, bool APPLY>
+// Block b of one tensor, U (one or two) heads side by side.  APPLY: codes
+// under the given scales; else the partial maxima, one per (head, row range).
+template <int D, int ROPE, bool APPLY, int U>
 __device__ __forceinline__ void rope_body(const PParams& p, int64_t b, uint32_t* partial,
                                           const float* dequant, int per_bh, uint8_t* codes) {
   constexpr int TPR = D / 16;                    // threads per row
   constexpr int RPI = kPThreads / TPR;           // rows per iteration
   constexpr int RPB = (int)(kPElemsPerBlock / D);
   static_assert(RPB % RPI == 0, "whole iterations");
-  constexpr int U = 2;                           // heads side by side
+  static_assert(U == 1 || U == 2, "heads side by side");
   __shared__ uint32_t s_max[kRopeMaxHeads];
   __shared__ float s_qm[kRopeMaxHeads];
   const RopeBlock rb = rope_block((uint32_t)b, (uint32_t)p.nsr, (uint32_t)p.nhc);
@@ -542,7 +550,9 @@ __device__ __forceinline__ void rope_body(const PParams& p, int64_t b, uint32_t*
 #pragma unroll 1
   for (int it = 0; it < RPB / RPI; ++it) {
     const int64_t s_own = sr * RPB + it * RPI + threadIdx.x / TPR;
-    if (sr * RPB + it * RPI >= p.S) break;
+    // a wave whose rows all lie past S leaves (no barrier in the loops)
+    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~(kWave - 1));
+    if (sr * RPB + it * RPI + wave0 / TPR >= p.S) break;
     const bool ok = s_own < p.S;
     const int64_t s = ok ? s_own : p.S - 1;      // read, never used
     float cs[16], sn[16];
@@ -577,12 +587,15 @@ __device__ __forceinline__ void rope_body(const PParams& p, int64_t b, uint32_t*
       if constexpr (!APPLY) {
         // both heads' maxima through one reduction, a 16-bit half each
         uint32_t v = 0;
-        if (ok) v = umax32(m[0] & 0xffffu, m[0] >> 16) | (umax32(m[1] & 0xffffu, m[1] >> 16) << 16);
+        if (ok) {
+          v = umax32(m[0] & 0xffffu, m[0] >> 16);
+          if constexpr (U == 2) v |= umax32(m[1] & 0xffffu, m[1] >> 16) << 16;
+        }
 #pragma unroll
         for (int o = 1; o <= 32; o <<= 1) v = pk_max_u16(v, (uint32_t)shfl_xor((int)v, o));
         if ((threadIdx.x & (kWave - 1)) == 0) {
           atomicMax(&s_max[h], v & 0xffffu);
-          atomicMax(&s_max[min(h + 1, nh - 1)], v >> 16);
+          if constexpr (U == 2) atomicMax(&s_max[min(h + 1, nh - 1)], v >> 16);
         }
       } else {
 #pragma unroll
@@ -621,13 +634,15 @@ __device__ __forceinline__ void rope_body(const PParams& p, int64_t b, uint32_t*
 template <int D, int ROPE>
 __device__ __forceinline__ void amax_block(const PParams& p, int64_t blk, uint32_t* partial) {
   if constexpr (ROPE == RP_ROPE_NONE) prologue_amax_body<D>(p, blk, partial);
-  else rope_body<D, ROPE, false>(p, blk, partial, nullptr, 0, nullptr);
+  else if (p.hc == 1) rope_body<D, ROPE, false, 1>(p, blk, partial, nullptr, 0, nullptr);
+  else rope_body<D, ROPE, false, 2>(p, blk, partial, nullptr, 0, nullptr);
 }
 template <int D, int ROPE>
 __device__ __forceinline__ void quant_block(const PParams& p, int64_t blk, const float* dequant,
                                             int per_bh, uint8_t* codes) {
   if constexpr (ROPE == RP_ROPE_NONE) prologue_quant_body<D>(p, blk, dequant, per_bh, codes);
-  else rope_body<D, ROPE, true>(p, blk, nullptr, dequant, per_bh, codes);
+  else if (p.hc == 1) rope_body<D, ROPE, true, 1>(p, blk, nullptr, dequant, per_bh, codes);
+  else rope_body<D, ROPE, true, 2>(p, blk, nullptr, dequant, per_bh, codes);
 }
 
 template <int D, int ROPE>
@@ -832,6 +847,7 @@ int make_pparams(const char* who, const void* x, int64_t B, int64_t H, int64_t S
     // the blocks cover the GPU several times over
     p.hc = kRopeHeads;
     while (p.hc > 2 && p.nsr * ((B * H + p.hc - 1) / p.hc) < kRopeMinBlocks) p.hc /= 2;
+    if (p.nsr * B * H <= kRopeSingleBlocks) p.hc = 1;
     p.nhc = (int)((B * H + p.hc - 1) / p.hc);
   }
   if (B * H > 0x7fffffffLL || 3 * max(ngroups * p.nbg, prologue_blocks(p, ngroups)) > 0x7fffffffLL) {
