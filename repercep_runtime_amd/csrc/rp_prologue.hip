@@ -413,21 +413,29 @@ __device__ __forceinline__ void prologue_quant_body(const PParams& p, int64_t bl
 // chunk per thread, 0.674 ms here; 4 or 16 heads per block 0.692 / 0.675 ms.
 constexpr int kRopeMaxHeads = 16;   // LDS words for a block's heads
 constexpr int kRopeHeads = 8;       // heads per block
-// Fewer heads per block, down to two, below this many blocks (per tensor): at
-// (1, 40, 16384, 128) 1024 and 256 take 0.264 and 0.267 ms, 3000 0.284 ms.
+// Heads per block by the number of (row range, head) pairs of a tensor: eight
+// where they leave 1024 blocks, else four, or two or one while those make at
+// most 341 blocks, 1024 for the call's three tensors -- then the chain of a
+// block's steps, not the tables' reads, is the call's time, and more blocks of
+// fewer heads shorten it as long as they all run at once.  Q, K and V from a
+// graph, us, a head per block and chunk per thread (before the tables were
+// kept in registers) / one, two, four, eight heads:
+//   40 (1, 40, 1, 128)     8.6 / 8.7, 9.8, -, -
+//  256 (4, 32, 256, 128)  35.1 / 23.6, 28.7, -, -
+//  360 (1, 40, 1152, 128) 43.4 / 33.2, 30.8, -, -
+//  512 (16, 32, 1, 128)   11.9 / 14.1, 12.7, 13.7, 18.5
+//  512 (8, 32, 256, 128)  46.9 / 47.0, 34.3, 47.3, 64.7
+//  672 (21, 32, 16, 128)  17.5 / 19.6, 16.1, 18.7, 22.1
+//  768 (2, 32, 1500, 128) 65.8 / 60.6, 52.8, 51.6, 81.8
+// 1024 (32, 32, 4, 128)   17.6 / 22.1, 19.5, 18.8, 22.4
+// 1024 (8, 32, 512, 128)  85.4 / 78.1, 68.0, 57.5, 86.4
+// 1760 (1, 16, 14000, 128) 945 / 618, 508, 483, 508
+// 2560 (1, 40, 8192, 128)  897 / 845, 688, 675, 683
+// Hundreds of heads of up to four positions each remain up to 7% behind the
+// first column.  At (1, 40, 16384, 128), 5120 pairs, four and eight heads take
+// 0.264 and 0.267 ms, two 0.284.
 constexpr int64_t kRopeMinBlocks = 1024;
-// One head per block while that makes at most this many blocks (per tensor):
-// the chain of one row's steps is such a call's time, and two heads side by
-// side only lengthen it.  A head per block and chunk per thread (before the
-// tables were kept in registers) / two heads / one, Q, K and V from a graph,
-// us: (1, 40, 1, 128) 8.6 / 9.8 / 8.7; (8, 32, 1, 128) 9.6 / 11.5 / 9.9;
-// (8, 32, 32, 64) 10.8 / 12.0 / 10.5; (1, 40, 512, 128) 33.1 / 22.7 / 21.0;
-// 256 blocks, (4, 32, 256, 128) 35.1 / 28.7 / 23.6; 320, (1, 32, 1280, 128)
-// 40.1 / 29.9 / 29.6; 360, (1, 40, 1152, 128) 43.4 / 30.8 / 33.2; 512,
-// (8, 32, 256, 128) 46.5 / 33.0 / 46.6.  More blocks of a few positions each
-// remain slower than they were: (16, 32, 1, 128) 11.8 / 12.7 / 13.9, (32, 32, 4,
-// 128) 18.0 / 19.4 / 22.2.
-constexpr int64_t kRopeSingleBlocks = 320;
+constexpr int64_t kRopeFewBlocks = 341;
 
 // two fp32 -> their nearest-even bf16 values as fp32 (one v_cvt_pk_bf16_f32)
 // and the packed pair
@@ -843,11 +851,10 @@ int make_pparams(const char* who, const void* x, int64_t B, int64_t H, int64_t S
   if (p.cosv != nullptr) {
     p.nsr = (S + p.rpb - 1) / p.rpb;
     p.nbg = p.nsr * (B * H / ngroups);
-    // heads per block: the more, the fewer reads of the tables, as long as
-    // the blocks cover the GPU several times over
-    p.hc = kRopeHeads;
-    while (p.hc > 2 && p.nsr * ((B * H + p.hc - 1) / p.hc) < kRopeMinBlocks) p.hc /= 2;
-    if (p.nsr * B * H <= kRopeSingleBlocks) p.hc = 1;
+    auto blocks = [&](int hc) { return p.nsr * ((B * H + hc - 1) / hc); };
+    p.hc = 4;
+    if (blocks(kRopeHeads) >= kRopeMinBlocks) p.hc = kRopeHeads;
+    else while (p.hc > 1 && blocks(p.hc / 2) <= kRopeFewBlocks) p.hc /= 2;
     p.nhc = (int)((B * H + p.hc - 1) / p.hc);
   }
   if (B * H > 0x7fffffffLL || 3 * max(ngroups * p.nbg, prologue_blocks(p, ngroups)) > 0x7fffffffLL) {

@@ -46,12 +46,14 @@ CASES = [
     ("per_tensor_short_heads", (2, 5, 3, 64), 1.0, False, "interleaved", "tensor"),
     ("short_heads_d128", (1, 7, 2, 128), 1.0, True, "half", "bh"),
     ("per_tensor_ragged", (3, 3, 37, 128), 1.0, True, None, "tensor"),
-    # rotary calls of (row ranges) x heads up to 320 run a head per block, one
-    # at a time; past it two side by side (an odd last head is repeated)
-    ("rope_320_heads", (1, 320, 9, 64), 1.0, True, "half", "bh"),
-    ("rope_321_heads", (1, 321, 9, 64), 1.0, True, "half", "bh"),
+    # rotary calls of (row ranges) x heads up to 341 run a head per block, one
+    # at a time; past it two or, past 682, four, two side by side (an odd last
+    # head is repeated)
+    ("rope_341_heads", (1, 341, 9, 64), 1.0, True, "half", "bh"),
+    ("rope_342_heads", (1, 342, 9, 64), 1.0, True, "half", "bh"),
+    ("rope_683_heads", (1, 683, 9, 64), 1.0, False, "interleaved", "bh"),
     ("rope_320_blocks_tensor", (1, 40, 1024, 128), 2.0, True, "interleaved", "tensor"),
-    ("rope_326_blocks", (1, 163, 200, 128), 2.0, False, "interleaved", "bh"),
+    ("rope_346_blocks", (1, 173, 200, 128), 2.0, False, "interleaved", "bh"),
     ("rope_410_blocks_tensor", (2, 41, 1100, 64), 2.0, True, "half", "tensor"),
 ]
 
@@ -244,8 +246,9 @@ def test_rotary_head_chunks_equal_single_heads(gpu: torch.device, rope: str, gra
     (1, 5, 1, 128, "half"),             # one row: one range, a head per block
     (2, 33, 300, 128, "interleaved"),   # three ranges, a head per block
     (3, 3, 2200, 64, "half"),           # nine ranges: a group of eight and one more
-    (2, 55, 300, 128, "half"),          # three ranges, 55 chunks of two heads
-    (1, 37, 2200, 64, "interleaved"),   # nine ranges, 19 chunks, the last of one head
+    (2, 59, 300, 128, "half"),          # three ranges, 59 chunks of two heads
+    (1, 39, 2200, 64, "interleaved"),   # nine ranges, 20 chunks, the last of one head
+    (1, 79, 2200, 64, "half"),          # nine ranges, 20 chunks of four, the last of three
 ])
 def test_rotary_few_ranges_equal_single_heads(gpu: torch.device, B: int, H: int, S: int, D: int,
                                               rope: str) -> None:
